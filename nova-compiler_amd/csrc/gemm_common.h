@@ -1,5 +1,5 @@
-// Device-side pieces shared by the two MFMA GEMM kernels (register-staged,
-// gemm_mfma.hip; LDS-DMA, gemm_dma.hip): argument block, MFMA wrapper,
+// Device-side pieces shared by the MFMA GEMM kernels (LDS-DMA: gemm_pers.h,
+// gemm_ring.h; register-staged: gemm_mfma.hip, gemm_small.hip): argument block, MFMA wrapper,
 // buffer resources, XCD-aware tile order and the bias / GELU / store
 // epilogue.
 #pragma once
@@ -211,52 +211,12 @@ __device__ __forceinline__ void store_outputs_t(const f32x16 (&acc)[TM][TN], con
   }
 }
 
-// The same with the output dtype and epilogue decided per element: smaller
-// code, used for large per-wave grids (4 x 4 tiles), where the specialised
-// form runs out of registers.
-template <int TM, int TN>
-__device__ __forceinline__ void store_outputs_any(const f32x16 (&acc)[TM][TN], const GemmArgs &a,
-                                                  int bidx, int mw, int nw, int lane) {
-  const int lrow = lane & 31, lhalf = lane >> 5;
-  char *Cb = static_cast<char *>(a.C) +
-             (int64_t)bidx * a.scb * (a.out_dt == NOVA_HIP_DT_F32 ? 4 : 2);
-  const bool has_bias = (a.epi == NOVA_HIP_EPI_BIAS || a.epi == NOVA_HIP_EPI_BIAS_GELU);
-  const bool has_gelu = (a.epi == NOVA_HIP_EPI_BIAS_GELU || a.epi == NOVA_HIP_EPI_GELU);
-#pragma unroll
-  for (int j = 0; j < TN; ++j) {
-    const int n = nw + j * 32 + lrow;
-    if (n >= a.N) continue;
-    const float bv = has_bias ? bias_at(a.bias, a.bias_dt, n) : 0.0f;
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int m = mw + i * 32 + 8 * (v >> 2) + 4 * lhalf + (v & 3);
-        if (m >= a.M) continue;
-        float x = acc[i][j][v];
-        if (has_bias) x = x + bv;
-        if (has_gelu) x = gelu_tanh(x);
-        const int64_t off = (int64_t)m * a.scm + n;
-        if (a.out_dt == NOVA_HIP_DT_F32)
-          reinterpret_cast<float *>(Cb)[off] = x;
-        else if (a.out_dt == NOVA_HIP_DT_BF16)
-          reinterpret_cast<uint16_t *>(Cb)[off] = to_bf16(x);
-        else
-          reinterpret_cast<uint16_t *>(Cb)[off] = to_f16(x);
-      }
-    }
-  }
-}
-
 // Runtime (output dtype, epilogue) -> one specialisation of store_outputs_t
 // (grids of up to 4 tiles per wave).
 template <int TM, int TN, bool NT = false>
 __device__ __forceinline__ void store_outputs(const f32x16 (&acc)[TM][TN], const GemmArgs &a,
                                               int bidx, int mw, int nw, int lane) {
-  if constexpr (TM * TN > 4) {
-    store_outputs_any<TM, TN>(acc, a, bidx, mw, nw, lane);
-    return;
-  }
+  static_assert(TM * TN <= 4, "larger grids run out of registers here");
   switch (a.out_dt * 4 + a.epi) {
 #define NOVA_EPI_CASE(O, E) \
   case O * 4 + E:           \
@@ -276,10 +236,11 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 }  // namespace gemm
 
-// Launchers (host).  launch_gemm_dma returns NOVA_HIP_EDTYPE when the
-// problem is not one the DMA kernel addresses (the caller then uses the
-// register-staged kernel).
-bool gemm_dma_applicable(const gemm::GemmArgs &a, bool akc, bool bkc, bool vec);
+// Launchers (host).  launch_gemm_aligned: problems with 16-byte aligned
+// operand rows, on the persistent kernel (gemm_pers.h, where it applies) or
+// a form of the ring kernel (gemm_ring.h).
+int32_t launch_gemm_aligned(const gemm::GemmArgs &a, int in_dt, bool akc, bool bkc, hipStream_t s);
+bool gemm_dma_applicable(const gemm::GemmArgs &a);
 int32_t launch_gemm_dma(const gemm::GemmArgs &a, int in_dt, bool akc, bool bkc, hipStream_t s);
 // Per output dtype (gemm_dma_out_{f32,bf16,f16}.hip, compiled separately).
 int32_t launch_gemm_dma_f32out(const gemm::GemmArgs &a, int in_dt, bool akc, bool bkc,

@@ -4,21 +4,21 @@
 // Replaces the NVPTX code generation of nova-gpu-optimized-pipeline for
 // linalg.matmul / linalg.batch_matmul (lib/Transforms/LLVMGPU/Passes.cpp:
 // 115-372: tile+distribute, pad, promote to shared memory, mma.sync,
-// 3-stage cp.async).  Two kernels, chosen per problem by launch_gemm_mfma:
+// 3-stage cp.async).  The kernels, chosen per problem by launch_gemm_mfma:
 //
-//  * gemm_dma.hip -- aligned problems made of whole 256x256x32 tiles (the
-//    large configs): operands go global -> LDS by DMA, four stages deep.
-//  * this file -- every other shape: register-staged loads, two LDS stages.
-//    Macro-tile BM x BN x 64, four wave64s in a 2x2 grid, each owning
-//    (BM/2) x (BN/2) of the output as 32x32 v_mfma_f32_32x32x16 tiles.
-//    LDS holds both operands K-contiguous ([rows][64] per stage) with the
-//    16-byte chunk index XOR-swizzled by row, so the ds_read_b128 of
-//    consecutive rows and the ds_write_b128 of one row's eight chunks hit
-//    distinct banks.  An operand whose unit stride is on M or N is
-//    fetched as 8x8 blocks and transposed in registers before the LDS
-//    write.  Edge tiles are zero-padded at load time (buffer loads outside
-//    the operand's range return zero) and masked at store time -- the role
-//    of NovaGPUPadOperands.
+//  * operands with 16-byte aligned rows: gemm_pers.h (whole 256x256 tiles,
+//    at least a round of them) and gemm_ring.h (every other shape);
+//  * unaligned rows: gemm_small.hip when the whole K of a tile fits LDS, else
+//    the kernel in this file: register-staged loads, two LDS stages.
+//    Macro-tile 64 x 64 x 64, four wave64s in a 2x2 grid, each owning one
+//    32x32 v_mfma_f32_32x32x16 tile.  LDS holds both operands K-contiguous
+//    ([rows][64] per stage) with the 16-byte chunk index XOR-swizzled by
+//    row, so the ds_read_b128 of consecutive rows and the ds_write_b128 of
+//    one row's eight chunks hit distinct banks.  An operand whose unit
+//    stride is on M or N is fetched as 8x8 blocks and transposed in
+//    registers before the LDS write.  Edge tiles are zero-padded at load
+//    time (buffer loads outside the operand's range return zero) and masked
+//    at store time -- the role of NovaGPUPadOperands.
 #include "gemm_common.h"
 
 namespace nova_hip {
@@ -41,8 +41,7 @@ __device__ __forceinline__ int lds_slot(int row, int c) {
 // any load outside it (edge rows, k past K, whole tiles past the end of the
 // K loop) returns zeros without touching memory, so edges need no branches.
 //   KC  : the operand's unit stride is on K.
-//   VEC : 16-byte loads are legal (16-byte aligned rows and chunks).
-//         Otherwise elements are fetched one by one (2-byte buffer loads).
+// Elements are fetched one by one (2-byte buffer loads).
 // ---------------------------------------------------------------------------
 template <int R, bool KC>
 struct TileShape {
@@ -59,15 +58,11 @@ struct Operand {
   int row0, rows, K;
 };
 
-__device__ __forceinline__ u32x4 load16(__amdgpu_buffer_rsrc_t r, uint32_t off) {
-  return __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0);
-}
-
 __device__ __forceinline__ uint32_t load2(__amdgpu_buffer_rsrc_t r, uint32_t off) {
   return (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(r, off, 0, 0);
 }
 
-template <int R, bool KC, bool VEC>
+template <int R, bool KC>
 __device__ __forceinline__ void load_tile(u32x4 *reg, const Operand &o, int k0, int tid) {
   if constexpr (KC) {
 #pragma unroll
@@ -76,19 +71,15 @@ __device__ __forceinline__ void load_tile(u32x4 *reg, const Operand &o, int k0, 
       const int r = q >> 3, c = q & 7;
       const int gr = o.row0 + r, gk = k0 + c * 8;
       const uint32_t base = (uint32_t)(((int64_t)gr * o.s_outer + gk) * 2);
-      if constexpr (VEC) {
-        reg[i] = load16(o.rsrc, (gr < o.rows && gk < o.K) ? base : kOOB);
-      } else {
-        uint32_t w[4];
+      uint32_t w[4];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const bool rok = gr < o.rows;
-          const uint32_t lo = load2(o.rsrc, (rok && gk + 2 * e < o.K) ? base + 4 * e : kOOB);
-          const uint32_t hi = load2(o.rsrc, (rok && gk + 2 * e + 1 < o.K) ? base + 4 * e + 2 : kOOB);
-          w[e] = lo | (hi << 16);
-        }
-        reg[i] = u32x4{w[0], w[1], w[2], w[3]};
+      for (int e = 0; e < 4; ++e) {
+        const bool rok = gr < o.rows;
+        const uint32_t lo = load2(o.rsrc, (rok && gk + 2 * e < o.K) ? base + 4 * e : kOOB);
+        const uint32_t hi = load2(o.rsrc, (rok && gk + 2 * e + 1 < o.K) ? base + 4 * e + 2 : kOOB);
+        w[e] = lo | (hi << 16);
       }
+      reg[i] = u32x4{w[0], w[1], w[2], w[3]};
     }
   } else {
     // 8x8 blocks: block q -> (rb = q / 8 row-block, kb = q % 8 k-block);
@@ -103,19 +94,15 @@ __device__ __forceinline__ void load_tile(u32x4 *reg, const Operand &o, int k0, 
       for (int j = 0; j < 8; ++j) {
         const int gk = k0 + kb * 8 + j;
         const uint32_t base = (uint32_t)(((int64_t)gk * o.s_outer + gr) * 2);
-        if constexpr (VEC) {
-          reg[it * 8 + j] = load16(o.rsrc, (qok && gk < o.K && gr < o.rows) ? base : kOOB);
-        } else {
-          uint32_t w[4];
+        uint32_t w[4];
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const bool kok = qok && gk < o.K;
-            const uint32_t lo = load2(o.rsrc, (kok && gr + 2 * e < o.rows) ? base + 4 * e : kOOB);
-            const uint32_t hi = load2(o.rsrc, (kok && gr + 2 * e + 1 < o.rows) ? base + 4 * e + 2 : kOOB);
-            w[e] = lo | (hi << 16);
-          }
-          reg[it * 8 + j] = u32x4{w[0], w[1], w[2], w[3]};
+        for (int e = 0; e < 4; ++e) {
+          const bool kok = qok && gk < o.K;
+          const uint32_t lo = load2(o.rsrc, (kok && gr + 2 * e < o.rows) ? base + 4 * e : kOOB);
+          const uint32_t hi = load2(o.rsrc, (kok && gr + 2 * e + 1 < o.rows) ? base + 4 * e + 2 : kOOB);
+          w[e] = lo | (hi << 16);
         }
+        reg[it * 8 + j] = u32x4{w[0], w[1], w[2], w[3]};
       }
     }
   }
@@ -152,7 +139,7 @@ __device__ __forceinline__ void store_tile(u32x4 *lds, const u32x4 *reg, int tid
   }
 }
 
-template <int DT, int BM, int BN, bool AKC, bool BKC, bool VEC>
+template <int DT, int BM, int BN, bool AKC, bool BKC>
 __global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(GemmArgs a) {
   constexpr int WTM = BM / 2, WTN = BN / 2;  // wave tile
   constexpr int TM = WTM / 32, TN = WTN / 32;
@@ -229,16 +216,16 @@ __global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(GemmArgs a) {
   // unconditional.
   u32x4 ra[SA::NREG], rb[SB::NREG];
   const int nk = (a.K + kBK - 1) / kBK;
-  load_tile<BM, AKC, VEC>(ra, oa, 0, tid);
-  load_tile<BN, BKC, VEC>(rb, ob, 0, tid);
+  load_tile<BM, AKC>(ra, oa, 0, tid);
+  load_tile<BN, BKC>(rb, ob, 0, tid);
   store_tile<BM, AKC>(lds_a[0], ra, tid);
   store_tile<BN, BKC>(lds_b[0], rb, tid);
   __syncthreads();
 
   for (int kt = 0; kt < nk; ++kt) {
     const int cur = kt & 1;
-    load_tile<BM, AKC, VEC>(ra, oa, (kt + 1) * kBK, tid);
-    load_tile<BN, BKC, VEC>(rb, ob, (kt + 1) * kBK, tid);
+    load_tile<BM, AKC>(ra, oa, (kt + 1) * kBK, tid);
+    load_tile<BN, BKC>(rb, ob, (kt + 1) * kBK, tid);
     __builtin_amdgcn_sched_barrier(0);
     compute(lds_a[cur], lds_b[cur]);
     store_tile<BM, AKC>(lds_a[cur ^ 1], ra, tid);
@@ -249,28 +236,21 @@ __global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(GemmArgs a) {
   store_outputs<TM, TN>(acc, a, bidx, m0 + wm * WTM, n0 + wn * WTN, lane);
 }
 
-template <int DT, int BM, int BN, bool AKC, bool BKC, bool VEC>
+template <int DT, int BM, int BN, bool AKC, bool BKC>
 int32_t launch_cfg(const GemmArgs &a, hipStream_t s) {
   const int64_t total = (int64_t)a.batch * a.tiles_m * a.tiles_n;
   if (total > 0x7fffffff) return fail(NOVA_HIP_ERANGE, "gemm: grid too large");
-  hipLaunchKernelGGL((gemm_mfma_kernel<DT, BM, BN, AKC, BKC, VEC>), dim3((unsigned)total),
+  hipLaunchKernelGGL((gemm_mfma_kernel<DT, BM, BN, AKC, BKC>), dim3((unsigned)total),
                      dim3(kThreads), 0, s, a);
   return check_hip(hipGetLastError(), "gemm_mfma launch");
 }
 
-template <int DT, int BM, int BN, bool VEC>
-int32_t dispatch_layout(const GemmArgs &a, bool akc, bool bkc, hipStream_t s) {
-  if (akc && bkc) return launch_cfg<DT, BM, BN, true, true, VEC>(a, s);
-  if (akc && !bkc) return launch_cfg<DT, BM, BN, true, false, VEC>(a, s);
-  if (!akc && bkc) return launch_cfg<DT, BM, BN, false, true, VEC>(a, s);
-  return launch_cfg<DT, BM, BN, false, false, VEC>(a, s);
-}
-
 template <int DT>
-int32_t dispatch_dtype(const GemmArgs &a, bool akc, bool bkc, bool big, bool vec, hipStream_t s) {
-  if (big) return dispatch_layout<DT, 256, 256, true>(a, akc, bkc, s);
-  if (vec) return dispatch_layout<DT, 64, 64, true>(a, akc, bkc, s);
-  return dispatch_layout<DT, 64, 64, false>(a, akc, bkc, s);
+int32_t dispatch_layout(const GemmArgs &a, bool akc, bool bkc, hipStream_t s) {
+  if (akc && bkc) return launch_cfg<DT, 64, 64, true, true>(a, s);
+  if (akc && !bkc) return launch_cfg<DT, 64, 64, true, false>(a, s);
+  if (!akc && bkc) return launch_cfg<DT, 64, 64, false, true>(a, s);
+  return launch_cfg<DT, 64, 64, false, false>(a, s);
 }
 
 bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
@@ -318,23 +298,17 @@ int32_t launch_gemm_mfma(const GemmProblem &p, hipStream_t s) {
   vec = vec && (p.a_kcontig ? (p.K % 8 == 0) : (p.M % 8 == 0));
   vec = vec && (p.b_kcontig ? (p.K % 8 == 0) : (p.N % 8 == 0));
 
-  if (gemm_dma_applicable(a, p.a_kcontig, p.b_kcontig, vec))
-    return launch_gemm_dma(a, p.in_dt, p.a_kcontig, p.b_kcontig, s);
+  if (vec) return launch_gemm_aligned(a, p.in_dt, p.a_kcontig, p.b_kcontig, s);
   // Rows without 16-byte alignment would cost the tiled kernel 2-byte loads;
   // with a small K the staged kernel copies them whole instead.
-  if (!vec && gemm_small_applicable(a, p.a_kcontig, p.b_kcontig))
+  if (gemm_small_applicable(a, p.a_kcontig, p.b_kcontig))
     return launch_gemm_small(a, p.in_dt, p.a_kcontig, p.b_kcontig, s);
 
-  // Tile choice: 256x256 when the grid still fills the chip, else 64x64.
-  const int64_t big_tiles = p.batch * ((p.M + 255) / 256) * ((p.N + 255) / 256);
-  const bool big = vec && big_tiles >= 256;
-  const int BMs = big ? 256 : 64;
-  a.tiles_m = (int)((p.M + BMs - 1) / BMs);
-  a.tiles_n = (int)((p.N + BMs - 1) / BMs);
-
+  a.tiles_m = (int)((p.M + 63) / 64);
+  a.tiles_n = (int)((p.N + 63) / 64);
   if (p.in_dt == NOVA_HIP_DT_BF16)
-    return dispatch_dtype<NOVA_HIP_DT_BF16>(a, p.a_kcontig, p.b_kcontig, big, vec, s);
-  return dispatch_dtype<NOVA_HIP_DT_F16>(a, p.a_kcontig, p.b_kcontig, big, vec, s);
+    return dispatch_layout<NOVA_HIP_DT_BF16>(a, p.a_kcontig, p.b_kcontig, s);
+  return dispatch_layout<NOVA_HIP_DT_F16>(a, p.a_kcontig, p.b_kcontig, s);
 }
 
 }  // namespace nova_hip

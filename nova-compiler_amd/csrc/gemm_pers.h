@@ -355,13 +355,6 @@ int32_t launch(const GemmArgs &a, hipStream_t s) {
   return check_hip(hipGetLastError(), "gemm_pers launch");
 }
 
-// The persistent kernel's problems: two K steps or more, a round size (one
-// workgroup per CU) and at least one full round of tiles.
-inline bool applicable(const GemmArgs &a) {
-  return a.K / BK >= 2 && a.round > 0 &&
-         (int64_t)a.batch * a.tiles_m * a.tiles_n >= a.round;
-}
-
 template <int ODT>
 int32_t launch_out(const GemmArgs &a, int in_dt, bool akc, bool bkc, hipStream_t s) {
   if (in_dt == NOVA_HIP_DT_BF16) {
