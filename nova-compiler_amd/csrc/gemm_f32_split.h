@@ -1,0 +1,656 @@
+// f32 GEMM on the bf16 matrix cores: each f32 value is the exact sum of
+// three bf16 values, x = h + m + l (8 + 8 + 8 significand bits; h and m are
+// rounded to nearest, so each remainder is at most 2^-9 of what it is a
+// remainder of), and a product a b is summed from six of the nine partial
+// products, h h, h m, m h, m m, h l, l h, on v_mfma_f32_32x32x16_bf16 with
+// f32 accumulation.  The three left out are below 2^-26 of the product, a
+// quarter of the rounding of an f32 multiply, and sixteen terms are summed
+// per accumulation instead of two, so the result is no further from the
+// exact sum than the f32 MFMA's.  Six bf16 MFMAs of this shape take 2.7
+// times fewer cycles than the eight v_mfma_f32_32x32x2_f32 they replace.
+//
+// Signs.  Where products reach below the accumulator's last bits (the small
+// partial products mostly do), the bf16 MFMA drops what is under its guard
+// bits towards minus infinity: a bias of one sign in every output (measured
+// mean -1.1e-6 of the outputs' scale at K = 50304 where plain bf16 operands
+// give -3e-9), harmless in an output but not in a sum of many outputs, such as
+// a bias gradient.  So every other unit of work, tiles and K splits counted
+// like the squares of a chess board, splits one operand with its sign changed,
+// sums the negated result and negates that.
+//
+// Length of a sum.  The MFMA also drops from each product what lies 2^-27 and
+// more below the accumulator, so where a few terms dwarf the others (a
+// one-hot gradient), small products lose bits that the f32 MFMA's fused
+// multiply-adds round in, the same way in every row.  So from K = 512 on a sum
+// is taken in at least three parts, of at most 3200 k: the K splits, and
+// within a split in chunks, each added in f32 to the output (or the split's
+// partial sum) by the workgroup that wrote it.  A sum over the rows of a loss
+// gradient times the head's weights, against 64 bits: 1.5e-6 off at 1000
+// classes in one part and 5.8e-7 in three (5.4e-7 on the f32 MFMA), 3.7e-6 at
+// 50304 classes in 8 parts and 1.1e-6 in 16 (1.5e-6 in 8 on the f32 MFMA).
+//
+// What bounds it: MFMA issue and the board's power limit.  A K step moves as
+// many bytes through LDS as a bf16 GEMM's and multiplies three times as long
+// on them, so two stages hide the DMA.  The splitting is VALU work (11
+// operations per pair of values) beside the MFMAs of the step before: it is
+// done as fragments are read, once per wave that needs one, which is why the
+// wave tiles are as large as the registers allow.
+//
+// Stages are those of gemm_ring.h with 32 f32 in place of 64 16-bit values:
+// a K-contiguous operand as [rows][8 chunks of 4 k], an M/N-contiguous one
+// as [32 k][rows / 4 chunks of 4 rows].  The latter is read with 4-byte
+// reads down the k-lines; its chunks are XOR-swizzled so that the two lane
+// halves, eight k-lines apart, fall on different banks.  Rows need only be
+// 4-byte aligned.
+//
+// Range.  A value beyond the largest bf16 splits into infinity and NaN, and
+// one below 2^-109 has bits under the smallest bf16.  A wave whose outputs
+// are not all finite, or of which one is non-zero but below 2^-96, computes
+// its tile again on v_mfma_f32_32x32x2_f32 straight from memory: infinities,
+// NaNs, overflow and underflow come out as f32 arithmetic gives them.
+#pragma once
+
+#include "gemm_ring.h"
+
+namespace nova_hip {
+namespace split {
+
+using namespace gemm;
+using dma::lds_addr;
+
+constexpr int BK = 32;
+// Parts that a sum of K terms is taken in, at least.
+inline int64_t min_parts(int64_t K) {
+  const int64_t n = (K + 3199) / 3200;
+  return K < 512 ? 1 : n < 3 ? 3 : n;
+}
+
+struct SplitArgs {
+  const float *A;
+  const float *B;
+  float *C;
+  const void *bias;
+  float *part;  // split-K partials [splits][batch][M][N], or null
+  int64_t sab, sa_outer, sbb, sb_outer, scb, scm;
+  uint32_t a_bytes, b_bytes;
+  int M, N, K;
+  int tiles_m, tiles_n, batch;
+  int splits, chunks;    // K in splits (workgroups) of chunks (units in turn)
+  int round;             // workgroups resident at once
+  int bias_dt, epi;
+};
+
+struct Pieces {
+  u32x4 p[3];  // h, m, l: eight bf16 each
+};
+
+// The eight values of a fragment (issued, not yet landed).
+struct Raw {
+  f32x4 v[2];
+};
+
+__device__ __forceinline__ float flip(float x, uint32_t sign) {
+  return __uint_as_float(__float_as_uint(x) ^ sign);
+}
+
+// Half of the splitting of values 2 q and 2 q + 1: h and the remainder
+// (unit 0), then m and l (unit 1).  FLIP: of the values with `sign` changed.
+template <bool FLIP>
+__device__ __forceinline__ void split_unit(Pieces &p, Raw &r, int q, int unit, uint32_t sign) {
+  float a = r.v[q >> 1][2 * (q & 1)], b = r.v[q >> 1][2 * (q & 1) + 1];
+  if (FLIP && unit == 0) {
+    a = flip(a, sign);
+    b = flip(b, sign);
+  }
+  const uint32_t w = pack_bf16(a, b);
+  a = a - __uint_as_float(w << 16);
+  b = b - __uint_as_float(w & 0xffff0000u);
+  p.p[unit][q] = w;
+  if (unit == 0) {
+    r.v[q >> 1][2 * (q & 1)] = a;
+    r.v[q >> 1][2 * (q & 1) + 1] = b;
+  } else {
+    p.p[2][q] = pack_bf16(a, b);
+  }
+}
+template <bool FLIP>
+__device__ __forceinline__ Pieces split8(Raw r, uint32_t sign) {
+  Pieces p;
+#pragma unroll
+  for (int u = 0; u < 8; ++u) split_unit<FLIP>(p, r, u >> 1, u & 1, sign);
+  return p;
+}
+
+// XOR of a chunk index of k-line k of an M/N-contiguous stage.
+__device__ __forceinline__ int line_swz(int k) { return (k & 8); }
+
+// Byte offset from the operand's stage base of this lane's first read of a
+// fragment (rows row_base + lane % 32, k = 16 kk + 8 (lane / 32) ... + 7).
+template <bool KC, int R>
+__device__ __forceinline__ uint32_t frag_offset(int row_base, int kk, int lane) {
+  const int row = row_base + (lane & 31), h = lane >> 5;
+  if constexpr (KC) {
+    return (uint32_t)(row * 8 + ((kk * 4 + h * 2) ^ ((row ^ (row >> 3)) & 7))) * 16u;
+  } else {
+    const int k = kk * 16 + h * 8;
+    return (uint32_t)(k * R + ((((row >> 2) ^ line_swz(k)) << 2) | (row & 3))) * 4u;
+  }
+}
+
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+template <int O0, int O1>
+__device__ __forceinline__ f32x2 lds_read2st64(uint32_t addr) {
+  f32x2 v;
+  asm volatile("ds_read2st64_b32 %0, %1 offset0:%2 offset1:%3" : "=v"(v) : "v"(addr), "n"(O0), "n"(O1));
+  return v;
+}
+template <bool KC, int R>
+__device__ __forceinline__ Raw read_raw(uint32_t addr) {
+  Raw r;
+  if constexpr (KC) {
+    r.v[0] = __builtin_bit_cast(f32x4, dma::lds_read_b128(addr));
+    r.v[1] = __builtin_bit_cast(f32x4, dma::lds_read_b128(addr ^ 16u));
+  } else {
+    constexpr int P = R / 64;  // a k-line in units of 64 dwords
+    const f32x2 a = lds_read2st64<0, P>(addr), b = lds_read2st64<2 * P, 3 * P>(addr);
+    const f32x2 c = lds_read2st64<4 * P, 5 * P>(addr), d = lds_read2st64<6 * P, 7 * P>(addr);
+    r.v[0] = f32x4{a[0], a[1], b[0], b[1]};
+    r.v[1] = f32x4{c[0], c[1], d[0], d[1]};
+  }
+  return r;
+}
+
+// In which phase of a k16 step (one per column block) each fragment of the
+// next step is read and split: about the same number in each, and B's block
+// j only after phase j has used its registers (the last goes to a spare set).
+template <int TM, int TN>
+constexpr int phase_of(int f) {
+  const int p = f >= TM ? f - TM + 1 : f < 2 ? 0 : f - 1;
+  return p < TN ? p : TN - 1;
+}
+// How many fragments phase j has, and which is its n-th.
+template <int TM, int TN>
+constexpr int phase_count(int j) {
+  int n = 0;
+  for (int f = 0; f < TM + TN; ++f) n += phase_of<TM, TN>(f) == j;
+  return n;
+}
+template <int TM, int TN>
+constexpr int phase_frag(int j, int n) {
+  for (int f = 0; f < TM + TN; ++f)
+    if (phase_of<TM, TN>(f) == j && n-- == 0) return f;
+  return -1;
+}
+
+// f(0), ..., f(N - 1) with constant arguments (a loop of this size is not
+// unrolled before the arrays in it must be registers).
+template <int N, typename Fn>
+__device__ __forceinline__ void static_for(Fn &&f) {
+  if constexpr (N > 0) {
+    static_for<N - 1>(f);
+    f(std::integral_constant<int, N - 1>{});
+  }
+}
+
+__device__ __forceinline__ f32x16 mfma_bf16(u32x4 a, u32x4 b, f32x16 c) {
+  return mfma_32x32x16<NOVA_HIP_DT_BF16>(a, b, c);
+}
+__device__ __forceinline__ void dma16(const float *p, uint32_t bytes, char *base, uint32_t off) {
+  ring::dma16(reinterpret_cast<const uint16_t *>(p), bytes, base, off);
+}
+__device__ __forceinline__ float load_f32(const float *p, uint32_t bytes, uint32_t off) {
+  return __builtin_bit_cast(
+      float, __builtin_amdgcn_raw_buffer_load_b32(
+                 make_rsrc(reinterpret_cast<const uint16_t *>(p), bytes), off, 0, 0));
+}
+
+// One unit of work: an output tile and the K steps [kt0, kt1) summed into it
+// (wave-uniform).  A tile's chunks of a split are consecutive units of one
+// workgroup.
+struct Tile {
+  int bidx, m0, n0, split, chunk, kt0, kt1;
+  uint32_t sign;  // the sign bit where the negated sum is taken, else 0
+};
+
+template <int BM, int BN>
+__device__ __forceinline__ Tile tile_at(const SplitArgs &a, int u) {
+  constexpr int G = 4;  // bands of G tile rows, swept column by column
+  const int tiles = a.batch * a.tiles_m * a.tiles_n;
+  const int ti = u / a.chunks, chunk = u - ti * a.chunks;
+  int id = blockIdx.x + ti * gridDim.x;
+  if (a.round > 0) id = ring::xcd_order(id, tiles * a.splits, a.round);
+  const int split = id / tiles;
+  id -= split * tiles;
+  const int per_batch = a.tiles_m * a.tiles_n;
+  const int bidx = id / per_batch;
+  const int t = id - bidx * per_batch;
+  const int band = t / (G * a.tiles_n), first = band * G;
+  const int gsz = min(a.tiles_m - first, G), in = t - band * G * a.tiles_n;
+  Tile r;
+  r.bidx = __builtin_amdgcn_readfirstlane(bidx);
+  r.m0 = __builtin_amdgcn_readfirstlane((first + in % gsz) * BM);
+  r.n0 = __builtin_amdgcn_readfirstlane(in / gsz * BN);
+  r.split = __builtin_amdgcn_readfirstlane(split);
+  r.chunk = __builtin_amdgcn_readfirstlane(chunk);
+  // K steps dealt out evenly over the splits' chunks.
+  const int64_t nk = (a.K + BK - 1) / BK, part = r.split * a.chunks + r.chunk;
+  const int64_t parts = (int64_t)a.splits * a.chunks;
+  r.kt0 = __builtin_amdgcn_readfirstlane((int)(part * nk / parts));
+  r.kt1 = __builtin_amdgcn_readfirstlane((int)((part + 1) * nk / parts));
+  r.sign = (uint32_t)__builtin_amdgcn_readfirstlane(
+      (int)((uint32_t)(first + in % gsz + in / gsz + split + chunk) << 31));
+  return r;
+}
+
+// 16 bytes to a row of any 4-byte alignment.
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+
+// Persistent: workgroup g of G computes tiles g, g + G, ... with the K steps
+// of all their units as one stream through the ring, so that the next
+// unit's first S steps are on their way (and its first fragments split)
+// before this one's outputs are written.  With more than one unit per
+// workgroup every unit has more than S steps (the steps being fetched when a
+// unit ends are then the next one's).
+template <bool AKC, bool BKC, int TM, int TN, int S>
+__global__ __launch_bounds__(kThreads) void gemm_f32_split_kernel(SplitArgs a) {
+  constexpr int BM = 64 * TM, BN = 64 * TN;
+  constexpr int LA = 2 * TM, LB = 2 * TN, L = LA + LB;
+  constexpr int kStageA = BM * BK * 4, kStage = (BM + BN) * BK * 4;
+  constexpr int F = TM + TN;
+  constexpr bool kFlipB = TN <= TM;  // the operand whose sign changes: the smaller
+  static_assert((S - 1) * L < 64, "vmcnt range");
+
+  __shared__ __attribute__((aligned(128))) char smem[S * kStage];
+  __shared__ f32x4 gelu_s[4][256];  // one 32 x 32 block per wave
+  static_assert(sizeof(smem) + sizeof(gelu_s) <= 160 * 1024, "LDS");
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int am = (wave >> 1) * 32 * TM, bn = (wave & 1) * 32 * TN;
+
+  const int total = a.batch * a.tiles_m * a.tiles_n * a.splits;
+  const int units = (total - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x * a.chunks;
+
+  // As in gemm_ring.h: byte offset (at k = 0, from the tile's first row) and
+  // k within a K step of the chunk this lane's DMA load i fetches.
+  auto setup = [&](auto kc, auto rows, int64_t s_outer, int i, uint32_t &off, int &kl)
+                   __attribute__((always_inline)) {
+    constexpr bool KC = decltype(kc)::value;
+    constexpr int CH = decltype(rows)::value / 4;
+    const int s = (i * 4 + wave) * 64 + lane;
+    if constexpr (KC) {
+      const int row = s >> 3, c = (s & 7) ^ ((row ^ (row >> 3)) & 7);
+      kl = c * 4;
+      off = (uint32_t)(((int64_t)row * s_outer + c * 4) * 4);
+    } else {
+      const int k = s / CH, c = (s - k * CH) ^ line_swz(k);
+      kl = k;
+      off = (uint32_t)(((int64_t)k * s_outer + c * 4) * 4);
+    }
+  };
+  uint32_t oa[LA], ob[LB];
+  int ka[LA], kb[LB];
+#pragma unroll
+  for (int i = 0; i < LA; ++i)
+    setup(std::integral_constant<bool, AKC>{}, std::integral_constant<int, BM>{}, a.sa_outer, i,
+          oa[i], ka[i]);
+#pragma unroll
+  for (int i = 0; i < LB; ++i)
+    setup(std::integral_constant<bool, BKC>{}, std::integral_constant<int, BN>{}, a.sb_outer, i,
+          ob[i], kb[i]);
+  // The next K step to fetch: S steps ahead of the one being multiplied.
+  struct {
+    const float *A, *B;   // batch slices
+    uint32_t at_a, at_b;  // byte offsets of the tile's K step
+    int left;             // K - k, or 0 with nothing to fetch
+    int steps;            // this unit's steps yet to fetch
+    int unit;
+    Tile t;
+  } next;
+  const uint32_t step_a = AKC ? BK * 4u : (uint32_t)(BK * a.sa_outer * 4);
+  const uint32_t step_b = BKC ? BK * 4u : (uint32_t)(BK * a.sb_outer * 4);
+  auto next_unit = [&](int u) __attribute__((always_inline)) {
+    next.unit = u;
+    next.left = next.steps = 0;
+    if (u >= units) return;
+    const Tile t = tile_at<BM, BN>(a, u);
+    next.t = t;
+    next.A = a.A + (int64_t)t.bidx * a.sab;
+    next.B = a.B + (int64_t)t.bidx * a.sbb;
+    next.at_a = (uint32_t)((AKC ? (int64_t)t.m0 * a.sa_outer : (int64_t)t.m0) * 4) + t.kt0 * step_a;
+    next.at_b = (uint32_t)((BKC ? (int64_t)t.n0 * a.sb_outer : (int64_t)t.n0) * 4) + t.kt0 * step_b;
+    next.steps = t.kt1 - t.kt0;
+    next.left = next.steps > 0 ? a.K - t.kt0 * BK : 0;
+  };
+  auto advance = [&]() __attribute__((always_inline)) {
+    next.at_a += step_a;
+    next.at_b += step_b;
+    next.left -= BK;
+    if (--next.steps <= 0) next_unit(next.unit + 1);
+  };
+  // DMA load q (A's first, then B's) of that step into stage st; nothing is
+  // read for k >= K.
+  auto dma = [&](int q, int st) __attribute__((always_inline)) {
+    char *base = smem + st * kStage;
+    if (q < LA)
+      dma16(next.A, a.a_bytes, base + (q * 4 + wave) * 1024,
+            ka[q] < next.left ? oa[q] + next.at_a : kOOB);
+    else
+      dma16(next.B, a.b_bytes, base + kStageA + ((q - LA) * 4 + wave) * 1024,
+            kb[q - LA] < next.left ? ob[q - LA] + next.at_b : kOOB);
+  };
+  // With K not a multiple of 4, the last chunk of a K-contiguous row holds
+  // values of the next row: zero them once the K step holding it has landed.
+  const bool tail = (AKC || BKC) && (a.K & 3) != 0;
+  auto zero_tail = [&](int st) __attribute__((always_inline)) {
+    const int kend = a.K & (BK - 1);
+    for (int r = tid; r < (AKC ? BM : 0) + (BKC ? BN : 0); r += kThreads) {
+      const int row = AKC && r >= BM ? r - BM : r;
+      float *base = reinterpret_cast<float *>(smem + st * kStage + ((AKC && r < BM) ? 0 : kStageA));
+      for (int k = kend; k & 3; ++k)
+        base[row * 32 + (((k >> 2) ^ ((row ^ (row >> 3)) & 7)) << 2) + (k & 3)] = 0.0f;
+    }
+    __syncthreads();
+  };
+
+  uint32_t fofs[2][F];
+#pragma unroll
+  for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+    for (int f = 0; f < F; ++f)
+      fofs[kk][f] = f < TM ? frag_offset<AKC, BM>(am + f * 32, kk, lane)
+                           : kStageA + frag_offset<BKC, BN>(bn + (f - TM) * 32, kk, lane);
+  const uint32_t lds0 = lds_addr(smem);
+  auto read_one = [&](int f, uint32_t stage, int kk) __attribute__((always_inline)) {
+    return f < TM ? read_raw<AKC, BM>(stage + fofs[kk][f]) : read_raw<BKC, BN>(stage + fofs[kk][f]);
+  };
+
+  f32x16 acc[TM][TN];
+  Pieces pa[2][TM], pb[TN], spare;
+
+  const int last_kt = (a.K + BK - 1) / BK - 1;  // the K step that may hold a tail
+
+  // Prologue: the first S steps in flight, the first landed and split.
+  next_unit(0);
+  Tile tc = next.t;
+#pragma unroll
+  for (int st = 0; st < S; ++st) {
+#pragma unroll
+    for (int q = 0; q < L; ++q) dma(q, st);
+    if (st < tc.kt1 - tc.kt0) advance();
+  }
+  NOVA_WAIT_VMCNT((S - 1) * L);
+  __builtin_amdgcn_s_barrier();
+  if (tail && tc.kt0 == last_kt) zero_tail(0);
+#pragma unroll
+  for (int f = 0; f < F; ++f) {
+    __builtin_amdgcn_sched_barrier(0);
+    const Raw r = read_one(f, lds0, 0);
+    NOVA_WAIT_LGKMCNT0();
+    __builtin_amdgcn_sched_barrier(0);
+    if (f < TM) pa[0][f] = split8<!kFlipB>(r, tc.sign);
+    else pb[f - TM] = split8<kFlipB>(r, tc.sign);
+  }
+
+  // One k16 step with A's pieces in pa[KK]: the MFMAs of column block j are
+  // phase j, the six partial products of each of its TM tiles, the smallest
+  // first; beside them the next step's fragments (k16 step KK ^ 1 at stage
+  // `from`) are read and split, the one operand with `sign` changed.  With
+  // KK = 1, the next K step is fetched into stage st meanwhile.
+  constexpr int kProd[6][2] = {{0, 2}, {2, 0}, {1, 1}, {0, 1}, {1, 0}, {0, 0}};
+  auto step = [&](auto kkc, uint32_t from, int st, uint32_t sign)
+                  __attribute__((always_inline)) {
+    constexpr int KK = decltype(kkc)::value;
+    static_for<TN>([&](auto jc) __attribute__((always_inline)) {
+      constexpr int j = decltype(jc)::value;
+      constexpr int NF = phase_count<TM, TN>(j);
+      __builtin_amdgcn_sched_barrier(0);
+      Raw raw[NF];
+      static_for<NF>([&](auto n) __attribute__((always_inline)) {
+        raw[n] = read_one(phase_frag<TM, TN>(j, n), from, KK ^ 1);
+      });
+      if constexpr (KK == 1) {
+        constexpr int kPer = (L + TN - 1) / TN;
+        static_for<kPer>([&](auto q) __attribute__((always_inline)) {
+          if constexpr (j * kPer + q < L) dma(j * kPer + q, st);
+        });
+      }
+      // MFMA m of the phase.
+      auto mfma_one = [&](int m) __attribute__((always_inline)) {
+        acc[m % TM][j] = mfma_bf16(pb[j].p[kProd[m / TM][1]], pa[KK][m % TM].p[kProd[m / TM][0]],
+                                   acc[m % TM][j]);
+      };
+      static_for<2 * TM>([&](auto m) __attribute__((always_inline)) { mfma_one(m); });
+      __builtin_amdgcn_sched_barrier(0);
+      NOVA_WAIT_LGKMCNT0();
+      __builtin_amdgcn_sched_barrier(0);
+      // The splitting goes out in units of five or six operations, spread
+      // evenly behind the 4 TM remaining MFMAs and fenced there.
+      constexpr int kMfma = 4 * TM, kUnits = 8 * NF;
+      Pieces nw[NF];
+      static_for<kMfma>([&](auto m) __attribute__((always_inline)) {
+        mfma_one(2 * TM + m);
+        constexpr int first = (m * kUnits + kMfma - 1) / kMfma;
+        constexpr int end = ((m + 1) * kUnits + kMfma - 1) / kMfma;
+        static_for<end - first>([&](auto v) __attribute__((always_inline)) {
+          constexpr int u = first + v;
+          constexpr bool isb = phase_frag<TM, TN>(j, u / 8) >= TM;
+          split_unit<isb == kFlipB>(nw[u / 8], raw[u / 8], (u % 8) >> 1, u & 1, sign);
+        });
+        __builtin_amdgcn_sched_barrier(0);
+      });
+      static_for<NF>([&](auto n) __attribute__((always_inline)) {
+        constexpr int f = phase_frag<TM, TN>(j, n);
+        // Opaque here: the compiler otherwise moves the whole step's
+        // splitting to the top of the next step, ahead of its MFMAs.
+        asm volatile("" : "+v"(nw[n].p[0]), "+v"(nw[n].p[1]), "+v"(nw[n].p[2]));
+        if constexpr (f < TM) pa[KK ^ 1][f] = nw[n];
+        else if constexpr (f - TM == j) spare = nw[n];
+        else pb[f - TM] = nw[n];
+      });
+    });
+    pb[TN - 1] = spare;
+  };
+
+  int cur = 0;
+  for (int ti = 0; ti < units; ++ti) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
+    for (int t = tc.kt0; t < tc.kt1; ++t) {
+      const int nxt = cur == S - 1 ? 0 : cur + 1;
+      step(std::integral_constant<int, 0>{}, lds0 + cur * kStage, 0, tc.sign);
+      // The next K step has landed for every wave, and nobody reads this
+      // one's stage any more: the step S on may go there.
+      __builtin_amdgcn_sched_barrier(0);
+      NOVA_WAIT_VMCNT((S - 2) * L);
+      __builtin_amdgcn_s_barrier();
+      if (tail && t + 1 == last_kt) zero_tail(nxt);
+      __builtin_amdgcn_sched_barrier(0);
+      step(std::integral_constant<int, 1>{}, lds0 + nxt * kStage, cur,
+           t + 1 < tc.kt1 ? tc.sign : next.t.sign);
+      advance();
+      cur = nxt;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+
+    // Outputs that the split does not represent: again in f32 (see the top).
+    // x * 0 is 0 or NaN; (x << 1) - 1 as an unsigned number orders by
+    // magnitude with zero on top.
+    // Values past the matrix's edges (whatever lies in memory there) do not
+    // count.
+    float fin = 0.0f;
+    uint32_t low = 0xffffffffu;
+    auto look = [&](float x) __attribute__((always_inline)) {
+      fin = __builtin_fmaf(x, 0.0f, fin);
+      low = min(low, (__float_as_uint(x) << 1) - 1u);
+    };
+    if (tc.m0 + BM <= a.M && tc.n0 + BN <= a.N) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+          for (int v = 0; v < 16; ++v) look(acc[i][j][v]);
+    } else {
+      const int rows = a.M - tc.m0 - am - (lane & 31), cols = a.N - tc.n0 - bn - 4 * (lane >> 5);
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+          for (int v = 0; v < 16; ++v)
+            look(32 * i < rows && 32 * j + 8 * (v >> 2) + (v & 3) < cols ? acc[i][j][v] : 0.0f);
+    }
+    constexpr uint32_t kTiny = (127u - 96u) << 24;  // 2^-96, shifted left by one
+    uint32_t sign = tc.sign;
+    if (__any(!(fin == 0.0f) || low < kTiny - 1u)) {
+      const float *Ab = a.A + (int64_t)tc.bidx * a.sab, *Bb = a.B + (int64_t)tc.bidx * a.sbb;
+      const int l32 = lane & 31, h = lane >> 5, kend = min(a.K, tc.kt1 * BK);
+      sign = 0;
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+          for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
+#pragma unroll 1
+      for (int k0 = tc.kt0 * BK; k0 < kend; k0 += 2) {
+        const int k = k0 + h;
+        float fa[TM], fb[TN];
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+          const int64_t m = tc.m0 + am + 32 * i + l32;
+          fa[i] = load_f32(Ab, a.a_bytes, k < kend && m < a.M
+              ? (uint32_t)((AKC ? m * a.sa_outer + k : k * a.sa_outer + m) * 4) : kOOB);
+        }
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          const int64_t n = tc.n0 + bn + 32 * j + l32;
+          fb[j] = load_f32(Bb, a.b_bytes, k < kend && n < a.N
+              ? (uint32_t)((BKC ? n * a.sb_outer + k : k * a.sb_outer + n) * 4) : kOOB);
+        }
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TN; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fb[j], fa[i], acc[i][j], 0, 0, 0);
+      }
+    }
+
+    // Outputs straight from the accumulators: lane l holds columns
+    // 8 g + 4 (l / 32) ... + 3 of row l % 32 of a block, 16 bytes.
+    const bool has_bias =
+        (a.epi == NOVA_HIP_EPI_BIAS || a.epi == NOVA_HIP_EPI_BIAS_GELU) && tc.kt0 == 0;
+    const bool has_gelu = (a.epi == NOVA_HIP_EPI_BIAS_GELU || a.epi == NOVA_HIP_EPI_GELU) &&
+                          !a.part && tc.kt1 * BK >= a.K;
+    float *Cb = a.part ? a.part + ((int64_t)tc.split * a.batch + tc.bidx) * a.M * a.N
+                       : a.C + (int64_t)tc.bidx * a.scb;
+    const int64_t ldc = a.part ? a.N : a.scm;
+    const int lr = lane & 31, lh = lane >> 5;
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      const int n = tc.n0 + bn + 32 * j + 4 * lh;
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[i][j][v] = flip(acc[i][j][v], sign);
+      if (has_bias) {
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float b = n + 8 * g + e < a.N ? bias_at(a.bias, a.bias_dt, n + 8 * g + e) : 0.0f;
+#pragma unroll
+            for (int i = 0; i < TM; ++i) acc[i][j][4 * g + e] += b;
+          }
+      }
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+        const int m = tc.m0 + am + 32 * i + lr;
+        float *row = Cb + (int64_t)m * ldc;
+        if (tc.chunk > 0 && m < a.M) {
+#pragma unroll
+          for (int g = 0; g < 4; ++g) {
+            const int c = n + 8 * g;
+            if (c + 4 <= a.N) {
+              const f32x4 old = *reinterpret_cast<const f32x4u *>(row + c);
+#pragma unroll
+              for (int e = 0; e < 4; ++e) acc[i][j][4 * g + e] += old[e];
+            } else {
+#pragma unroll
+              for (int e = 0; e < 3; ++e)
+                if (c + e < a.N) acc[i][j][4 * g + e] += row[c + e];
+            }
+          }
+        }
+        if (has_gelu) {  // tanhf is large: in a rolled loop, through LDS
+          f32x4 *blk = gelu_s[wave];
+#pragma unroll
+          for (int g = 0; g < 4; ++g)
+            blk[g * 64 + lane] = f32x4{acc[i][j][4 * g], acc[i][j][4 * g + 1],
+                                       acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
+#pragma unroll 1
+          for (int g = 0; g < 4; ++g) {
+            f32x4 x = blk[g * 64 + lane];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[e] = gelu_tanh(x[e]);
+            blk[g * 64 + lane] = x;
+          }
+#pragma unroll
+          for (int g = 0; g < 4; ++g) {
+            const f32x4 x = blk[g * 64 + lane];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[i][j][4 * g + e] = x[e];
+          }
+        }
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const int c = n + 8 * g;
+          if (m < a.M && c + 4 <= a.N) {
+            *reinterpret_cast<f32x4u *>(row + c) = f32x4{acc[i][j][4 * g], acc[i][j][4 * g + 1],
+                                                         acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
+          } else if (m < a.M) {
+#pragma unroll
+            for (int e = 0; e < 3; ++e)
+              if (c + e < a.N) row[c + e] = acc[i][j][4 * g + e];
+          }
+        }
+      }
+    }
+    tc = next.t;
+  }
+  NOVA_WAIT_VMCNT(0);  // no DMA may target this workgroup's LDS when it retires
+}
+
+// The tile forms (launch_form's cases, in this order) and what the choice
+// between them (gemm_f32_mfma.hip) needs to know of each.
+struct Form {
+  int tm, tn, stages, per_cu;  // tile 64 tm x 64 tn; workgroups per CU
+  float step, more, fixed;     // us: see estimate()
+};
+constexpr int kForms = 6;
+
+template <bool AKC, bool BKC>
+int32_t launch_form(int form, const SplitArgs &r, unsigned grid, hipStream_t s) {
+  const dim3 g(grid), b(kThreads);
+  switch (form) {
+    case 0: hipLaunchKernelGGL((gemm_f32_split_kernel<AKC, BKC, 4, 3, 2>), g, b, 0, s, r); break;
+    case 1: hipLaunchKernelGGL((gemm_f32_split_kernel<AKC, BKC, 3, 4, 2>), g, b, 0, s, r); break;
+    case 2: hipLaunchKernelGGL((gemm_f32_split_kernel<AKC, BKC, 3, 3, 2>), g, b, 0, s, r); break;
+    case 3: hipLaunchKernelGGL((gemm_f32_split_kernel<AKC, BKC, 4, 2, 2>), g, b, 0, s, r); break;
+    case 4: hipLaunchKernelGGL((gemm_f32_split_kernel<AKC, BKC, 2, 2, 2>), g, b, 0, s, r); break;
+    default: hipLaunchKernelGGL((gemm_f32_split_kernel<AKC, BKC, 1, 1, 3>), g, b, 0, s, r); break;
+  }
+  return check_hip(hipGetLastError(), "gemm_f32_split launch");
+}
+
+// By A's layout (gemm_f32_split_{kc,mc}.hip, compiled in parallel).
+int32_t launch_a_kcontig(int form, const SplitArgs &r, bool bkc, unsigned grid, hipStream_t s);
+int32_t launch_a_mcontig(int form, const SplitArgs &r, bool bkc, unsigned grid, hipStream_t s);
+
+}  // namespace split
+}  // namespace nova_hip
