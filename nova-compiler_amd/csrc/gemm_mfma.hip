@@ -9,17 +9,20 @@
 //  * operands with 16-byte aligned rows: gemm_pers.h (whole 256x256 tiles,
 //    at least a round of them) and gemm_ring.h (every other shape);
 //  * unaligned rows: gemm_small.hip when the whole K of a tile fits LDS, else
-//    the kernel in this file: register-staged loads, two LDS stages.
-//    Macro-tile 64 x 64 x 64, four wave64s in a 2x2 grid, each owning one
-//    32x32 v_mfma_f32_32x32x16 tile.  LDS holds both operands K-contiguous
-//    ([rows][64] per stage) with the 16-byte chunk index XOR-swizzled by
-//    row, so the ds_read_b128 of consecutive rows and the ds_write_b128 of
-//    one row's eight chunks hit distinct banks.  An operand whose unit
-//    stride is on M or N is fetched as 8x8 blocks and transposed in
-//    registers before the LDS write.  Edge tiles are zero-padded at load
-//    time (buffer loads outside the operand's range return zero) and masked
-//    at store time -- the role of NovaGPUPadOperands.
-#include "gemm_common.h"
+//    the kernel in this file.
+//
+// gemm_unaligned_kernel: rows at any 2-byte alignment.  What bounded its
+// predecessor was its loads, one element each.  LDS DMA cannot shift, so each
+// 16-byte chunk goes through registers: the four dwords that hold its first
+// byte and the dword behind them (both dword-aligned, so legal for any
+// element), shifted together by the row's odd half dword.  The chunk's shift
+// is the same in every K step, as a step is a multiple of four bytes in
+// either layout.  Stages, swizzles and fragment reads are those of
+// gemm_ring.h, two stages deep with the next step's loads in registers; tile
+// 64 T x 64 T, four waves.  Edge tiles as there: rows past M or N feed only
+// outputs that are not stored (the resource covers the slice, out to dword
+// boundaries), k past K reads zero.
+#include "gemm_ring.h"
 
 namespace nova_hip {
 namespace {
@@ -28,229 +31,189 @@ using namespace gemm;
 
 constexpr int kBK = 64;  // K per LDS stage
 
-// LDS chunk slot of (row, 16-byte chunk c) inside one operand stage.  The
-// XOR by (row ^ row/8) keeps both 8 and 16 consecutive rows of a
-// ds_read_b128 on distinct banks (LDS serving 8 or 16 lanes per cycle).
-__device__ __forceinline__ int lds_slot(int row, int c) {
-  return row * 8 + (c ^ ((row ^ (row >> 3)) & 7));
-}
-
-// ---------------------------------------------------------------------------
-// Tile loaders.  An operand tile is R rows (M for A, N for B) x 64 k, read
-// through a buffer resource whose range covers the operand's batch slice:
-// any load outside it (edge rows, k past K, whole tiles past the end of the
-// K loop) returns zeros without touching memory, so edges need no branches.
-//   KC  : the operand's unit stride is on K.
-// Elements are fetched one by one (2-byte buffer loads).
-// ---------------------------------------------------------------------------
-template <int R, bool KC>
-struct TileShape {
-  // KC: R*8 chunks over 256 threads.  !KC: R blocks of 8x8, one block
-  // (8 chunks) per participating thread.
-  static constexpr int kBlocks = KC ? 0 : R;
-  static constexpr int kBlockIters = KC ? 0 : (kBlocks + kThreads - 1) / kThreads;
-  static constexpr int NREG = KC ? (R * 8) / kThreads : 8 * kBlockIters;
+struct Chunk {
+  u32x4 lo;
+  uint32_t hi;
 };
 
-struct Operand {
+__device__ __forceinline__ Chunk load_chunk(__amdgpu_buffer_rsrc_t r, uint32_t off) {
+  return Chunk{__builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0),
+               (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(r, off, 16, 0)};
+}
+
+// The chunk's eight elements, with only the first `left` kept.
+__device__ __forceinline__ u32x4 shifted(const Chunk &c, uint32_t shift, int left) {
+  u32x4 v;
+#pragma unroll
+  for (int d = 0; d < 4; ++d) {
+    const uint32_t w = __builtin_amdgcn_alignbyte(d < 3 ? c.lo[d < 3 ? d + 1 : 3] : c.hi, c.lo[d], shift);
+    v[d] = 2 * d + 1 < left ? w : 2 * d < left ? w & 0xffffu : 0u;
+  }
+  return v;
+}
+
+// A fragment of gemm_ring.h's stages (rows row_base + lane % 32, k16 step kk).
+template <bool KC, int R>
+__device__ __forceinline__ u32x4 read_frag(const char *stage, int row_base, int kk, int lane) {
+  const char *p = stage + ring::frag_offset<KC, R>(row_base, kk, lane);
+  if constexpr (KC) {
+    return *reinterpret_cast<const u32x4 *>(p);
+  } else {
+    typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
+    const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4 *)p);
+    const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4 *)(p + 4 * R * 2));
+    const u32x2 l = __builtin_bit_cast(u32x2, lo), h = __builtin_bit_cast(u32x2, hi);
+    return u32x4{l[0], l[1], h[0], h[1]};
+  }
+}
+
+// One operand's loads: chunk i of a thread is slot (i * 256 + tid) of the
+// stage.  off: byte offset at k = 0 from the dword that holds the slice's
+// first element.
+template <bool KC, int R>
+struct Loader {
+  static constexpr int kN = R * 8 / kThreads, CH = R / 8;
   __amdgpu_buffer_rsrc_t rsrc;
-  int64_t s_outer;  // elements
-  int row0, rows, K;
+  uint32_t off[kN];
+  uint32_t step;
+  Chunk c[kN];
+
+  __device__ __forceinline__ static int k_of(int i) {  // the chunk's k within a step
+    const int s = i * kThreads + (int)threadIdx.x;
+    if constexpr (KC) {
+      const int row = s >> 3;
+      return ((s & 7) ^ ((row ^ (row >> 3)) & 7)) * 8;
+    } else {
+      return s / CH;
+    }
+  }
+  __device__ __forceinline__ void init(const uint16_t *p, uint32_t bytes, int row0, int64_t s_outer) {
+    const uint32_t mis = (uint32_t)(reinterpret_cast<uintptr_t>(p) & 2u);
+    rsrc = make_rsrc(reinterpret_cast<const uint16_t *>(reinterpret_cast<uintptr_t>(p) - mis),
+                     bytes ? (bytes + mis + 3u) & ~3u : 0u);
+    step = KC ? kBK * 2u : (uint32_t)(kBK * s_outer * 2);
+#pragma unroll
+    for (int i = 0; i < kN; ++i) {
+      const int s = i * kThreads + (int)threadIdx.x, k = k_of(i);
+      const int64_t e = KC ? (int64_t)(row0 + (s >> 3)) * s_outer + k
+                           : (int64_t)k * s_outer + row0 +
+                                 (((s % CH) ^ ring::line_swz<CH>(k)) * 8);
+      off[i] = mis + (uint32_t)(e * 2);
+    }
+  }
+  __device__ __forceinline__ void load(int kt, int K) {
+#pragma unroll
+    for (int i = 0; i < kN; ++i)
+      c[i] = load_chunk(rsrc, k_of(i) < K - kt * kBK ? (off[i] & ~3u) + (uint32_t)kt * step : kOOB);
+  }
+  __device__ __forceinline__ void store(char *stage, int kt, int K) const {
+#pragma unroll
+    for (int i = 0; i < kN; ++i) {
+      const int left = KC ? K - kt * kBK - k_of(i) : 8;
+      reinterpret_cast<u32x4 *>(stage)[i * kThreads + threadIdx.x] = shifted(c[i], off[i] & 2u, left);
+    }
+  }
 };
 
-__device__ __forceinline__ uint32_t load2(__amdgpu_buffer_rsrc_t r, uint32_t off) {
-  return (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(r, off, 0, 0);
-}
+template <int DT, bool AKC, bool BKC, int T>
+__global__ __launch_bounds__(kThreads) void gemm_unaligned_kernel(GemmArgs a, int vec_out) {
+  constexpr int B = 64 * T, kStageA = B * kBK * 2, kStage = 2 * kStageA;
+  __shared__ __attribute__((aligned(16))) char smem[2 * kStage];
+  __shared__ __attribute__((aligned(16))) float bias_s[B];
 
-template <int R, bool KC>
-__device__ __forceinline__ void load_tile(u32x4 *reg, const Operand &o, int k0, int tid) {
-  if constexpr (KC) {
-#pragma unroll
-    for (int i = 0; i < TileShape<R, KC>::NREG; ++i) {
-      const int q = tid + i * kThreads;
-      const int r = q >> 3, c = q & 7;
-      const int gr = o.row0 + r, gk = k0 + c * 8;
-      const uint32_t base = (uint32_t)(((int64_t)gr * o.s_outer + gk) * 2);
-      uint32_t w[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const bool rok = gr < o.rows;
-        const uint32_t lo = load2(o.rsrc, (rok && gk + 2 * e < o.K) ? base + 4 * e : kOOB);
-        const uint32_t hi = load2(o.rsrc, (rok && gk + 2 * e + 1 < o.K) ? base + 4 * e + 2 : kOOB);
-        w[e] = lo | (hi << 16);
-      }
-      reg[i] = u32x4{w[0], w[1], w[2], w[3]};
-    }
-  } else {
-    // 8x8 blocks: block q -> (rb = q / 8 row-block, kb = q % 8 k-block);
-    // chunk j of the block holds k-row (kb*8 + j), rows rb*8 .. rb*8+7.
-#pragma unroll
-    for (int it = 0; it < TileShape<R, KC>::kBlockIters; ++it) {
-      const int q = tid + it * kThreads;
-      const int kb = q & 7, rb = q >> 3;
-      const int gr = o.row0 + rb * 8;
-      const bool qok = q < TileShape<R, KC>::kBlocks;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const int gk = k0 + kb * 8 + j;
-        const uint32_t base = (uint32_t)(((int64_t)gk * o.s_outer + gr) * 2);
-        uint32_t w[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const bool kok = qok && gk < o.K;
-          const uint32_t lo = load2(o.rsrc, (kok && gr + 2 * e < o.rows) ? base + 4 * e : kOOB);
-          const uint32_t hi = load2(o.rsrc, (kok && gr + 2 * e + 1 < o.rows) ? base + 4 * e + 2 : kOOB);
-          w[e] = lo | (hi << 16);
-        }
-        reg[it * 8 + j] = u32x4{w[0], w[1], w[2], w[3]};
-      }
-    }
-  }
-}
-
-template <int R, bool KC>
-__device__ __forceinline__ void store_tile(u32x4 *lds, const u32x4 *reg, int tid) {
-  if constexpr (KC) {
-#pragma unroll
-    for (int i = 0; i < TileShape<R, KC>::NREG; ++i) {
-      const int q = tid + i * kThreads;
-      lds[lds_slot(q >> 3, q & 7)] = reg[i];
-    }
-  } else {
-#pragma unroll
-    for (int it = 0; it < TileShape<R, KC>::kBlockIters; ++it) {
-      const int q = tid + it * kThreads;
-      if (q >= TileShape<R, KC>::kBlocks) break;
-      const int kb = q & 7, rb = q >> 3;
-      const u32x4 *in = reg + it * 8;  // in[j]: k-row j, 8 values along rows
-      // Transpose: output row r (0..7) gathers element r of each k-row.
-#pragma unroll
-      for (int r = 0; r < 8; ++r) {
-        const int d = r >> 1;
-        uint32_t w[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const uint32_t x = in[2 * e][d], y = in[2 * e + 1][d];
-          w[e] = (r & 1) ? ((x >> 16) | (y & 0xffff0000u)) : ((x & 0xffffu) | (y << 16));
-        }
-        lds[lds_slot(rb * 8 + r, kb)] = u32x4{w[0], w[1], w[2], w[3]};
-      }
-    }
-  }
-}
-
-template <int DT, int BM, int BN, bool AKC, bool BKC>
-__global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(GemmArgs a) {
-  constexpr int WTM = BM / 2, WTN = BN / 2;  // wave tile
-  constexpr int TM = WTM / 32, TN = WTN / 32;
-  using SA = TileShape<BM, AKC>;
-  using SB = TileShape<BN, BKC>;
-
-  __shared__ u32x4 lds_a[2][BM * 8];
-  __shared__ u32x4 lds_b[2][BN * 8];
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int am = (wave >> 1) * 32 * T, bn = (wave & 1) * 32 * T;
   int bidx, tm, tn;
   tile_of(blockIdx.x, a, bidx, tm, tn);
-  const int m0 = tm * BM, n0 = tn * BN;
+  const int m0 = tm * B, n0 = tn * B;
+  const bool has_bias = (a.epi == NOVA_HIP_EPI_BIAS || a.epi == NOVA_HIP_EPI_BIAS_GELU);
+  const bool has_gelu = (a.epi == NOVA_HIP_EPI_BIAS_GELU || a.epi == NOVA_HIP_EPI_GELU);
+  if (has_bias && tid < B) bias_s[tid] = n0 + tid < a.N ? bias_at(a.bias, a.bias_dt, n0 + tid) : 0.f;
 
-  Operand oa, ob;
-  oa.rsrc = make_rsrc(a.A + (int64_t)bidx * a.sab, a.a_bytes);
-  oa.s_outer = a.sa_outer;
-  oa.row0 = m0;
-  oa.rows = a.M;
-  oa.K = a.K;
-  ob.rsrc = make_rsrc(a.B + (int64_t)bidx * a.sbb, a.b_bytes);
-  ob.s_outer = a.sb_outer;
-  ob.row0 = n0;
-  ob.rows = a.N;
-  ob.K = a.K;
+  Loader<AKC, B> la;
+  Loader<BKC, B> lb;
+  la.init(a.A + (int64_t)bidx * a.sab, a.a_bytes, m0, a.sa_outer);
+  lb.init(a.B + (int64_t)bidx * a.sbb, a.b_bytes, n0, a.sb_outer);
 
-  f32x16 acc[TM][TN];
+  f32x16 acc[T][T];
 #pragma unroll
-  for (int i = 0; i < TM; ++i)
+  for (int i = 0; i < T; ++i)
 #pragma unroll
-    for (int j = 0; j < TN; ++j)
+    for (int j = 0; j < T; ++j)
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
 
-  const int lrow = lane & 31;   // row (A) / column (B) inside a 32-tile
-  const int lhalf = lane >> 5;  // which 8-wide k half of a 16-k step
-
-  // One LDS stage through the MFMAs; fragments of step kk+1 are read while
-  // the MFMAs of step kk run.  The scheduling barriers keep that order: left
-  // alone, the scheduler sinks reads next to their first use to save
-  // registers and exposes the LDS latency at every step.
-  auto compute = [&](const u32x4 *sa, const u32x4 *sb) __attribute__((always_inline)) {
-    u32x4 fa[2][TM], fb[2][TN];
-#pragma unroll
-    for (int i = 0; i < TM; ++i) fa[0][i] = sa[lds_slot(wm * WTM + i * 32 + lrow, lhalf)];
-#pragma unroll
-    for (int j = 0; j < TN; ++j) fb[0][j] = sb[lds_slot(wn * WTN + j * 32 + lrow, lhalf)];
+  const int nk = (a.K + kBK - 1) / kBK;
+  la.load(0, a.K);
+  lb.load(0, a.K);
+  la.store(smem, 0, a.K);
+  lb.store(smem + kStageA, 0, a.K);
+  la.load(1, a.K);
+  lb.load(1, a.K);
+  __syncthreads();
+  for (int kt = 0; kt < nk; ++kt) {
+    const char *cur = smem + (kt & 1) * kStage;
+    char *nxt = smem + ((kt & 1) ^ 1) * kStage;
+    // The step after this one, loaded a step ago, into the other stage (free
+    // since the last barrier), and the loads of the one after that.
+    if (kt + 1 < nk) {
+      la.store(nxt, kt + 1, a.K);
+      lb.store(nxt + kStageA, kt + 1, a.K);
+      la.load(kt + 2, a.K);
+      lb.load(kt + 2, a.K);
+    }
 #pragma unroll
     for (int kk = 0; kk < kBK / 16; ++kk) {
-      const int cb = kk & 1, nb = cb ^ 1;
-      if (kk + 1 < kBK / 16) {
-        const int chunk = (kk + 1) * 2 + lhalf;
+      u32x4 fa[T], fb[T];
 #pragma unroll
-        for (int i = 0; i < TM; ++i) fa[nb][i] = sa[lds_slot(wm * WTM + i * 32 + lrow, chunk)];
+      for (int i = 0; i < T; ++i) fa[i] = read_frag<AKC, B>(cur, am + i * 32, kk, lane);
 #pragma unroll
-        for (int j = 0; j < TN; ++j) fb[nb][j] = sb[lds_slot(wn * WTN + j * 32 + lrow, chunk)];
-      }
-      __builtin_amdgcn_sched_barrier(0);
+      for (int j = 0; j < T; ++j) fb[j] = read_frag<BKC, B>(cur + kStageA, bn + j * 32, kk, lane);
 #pragma unroll
-      for (int i = 0; i < TM; ++i)
+      for (int i = 0; i < T; ++i)
 #pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] = mfma_32x32x16<DT>(fa[cb][i], fb[cb][j], acc[i][j]);
-      __builtin_amdgcn_sched_barrier(0);
+        for (int j = 0; j < T; ++j) acc[i][j] = mfma_32x32x16<DT>(fb[j], fa[i], acc[i][j]);
     }
-  };
-
-  // The global loads of tile t+1 are issued before the MFMAs of tile t and
-  // written to the other LDS stage after them.  Loads past the last tile
-  // fall outside the buffer range and return zeros, so the loop body is
-  // unconditional.
-  u32x4 ra[SA::NREG], rb[SB::NREG];
-  const int nk = (a.K + kBK - 1) / kBK;
-  load_tile<BM, AKC>(ra, oa, 0, tid);
-  load_tile<BN, BKC>(rb, ob, 0, tid);
-  store_tile<BM, AKC>(lds_a[0], ra, tid);
-  store_tile<BN, BKC>(lds_b[0], rb, tid);
-  __syncthreads();
-
-  for (int kt = 0; kt < nk; ++kt) {
-    const int cur = kt & 1;
-    load_tile<BM, AKC>(ra, oa, (kt + 1) * kBK, tid);
-    load_tile<BN, BKC>(rb, ob, (kt + 1) * kBK, tid);
-    __builtin_amdgcn_sched_barrier(0);
-    compute(lds_a[cur], lds_b[cur]);
-    store_tile<BM, AKC>(lds_a[cur ^ 1], ra, tid);
-    store_tile<BN, BKC>(lds_b[cur ^ 1], rb, tid);
     __syncthreads();
   }
 
-  store_outputs<TM, TN>(acc, a, bidx, m0 + wm * WTM, n0 + wn * WTN, lane);
+  char *stg = smem + wave * (32 * 32 * T * 4);
+  const float *bias_w = has_bias ? bias_s + bn : nullptr;
+  const int lr = lane & 31, lh = lane >> 5;
+#pragma unroll
+  for (int i = 0; i < T; ++i) {
+#pragma unroll
+    for (int j = 0; j < T; ++j)
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        *ring::stage_chunk<32 * T>(stg, lr, 8 * j + 2 * g + lh) = f32x4{
+            acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
+    const int mb = m0 + am + 32 * i, nw = n0 + bn;
+    const int64_t at = (int64_t)bidx * a.scb + (int64_t)mb * a.scm + nw;
+    if (a.out_dt == NOVA_HIP_DT_F32)
+      ring::store_f32<32, 32 * T, 64, 1>(stg, 0, lane, static_cast<float *>(a.C) + at, a.scm,
+                                         a.M - mb, a.N - nw, vec_out, bias_w, has_gelu);
+    else
+      ring::store_16<32, 32 * T, 64, 1>(stg, 0, lane, static_cast<uint16_t *>(a.C) + at, a.scm,
+                                        a.M - mb, a.N - nw, vec_out, bias_w, has_gelu,
+                                        a.out_dt == NOVA_HIP_DT_BF16);
+  }
 }
 
-template <int DT, int BM, int BN, bool AKC, bool BKC>
-int32_t launch_cfg(const GemmArgs &a, hipStream_t s) {
+template <int DT, int T>
+int32_t launch_cfg(const GemmArgs &a, int vec_out, bool akc, bool bkc, hipStream_t s) {
   const int64_t total = (int64_t)a.batch * a.tiles_m * a.tiles_n;
   if (total > 0x7fffffff) return fail(NOVA_HIP_ERANGE, "gemm: grid too large");
-  hipLaunchKernelGGL((gemm_mfma_kernel<DT, BM, BN, AKC, BKC>), dim3((unsigned)total),
-                     dim3(kThreads), 0, s, a);
-  return check_hip(hipGetLastError(), "gemm_mfma launch");
-}
-
-template <int DT>
-int32_t dispatch_layout(const GemmArgs &a, bool akc, bool bkc, hipStream_t s) {
-  if (akc && bkc) return launch_cfg<DT, 64, 64, true, true>(a, s);
-  if (akc && !bkc) return launch_cfg<DT, 64, 64, true, false>(a, s);
-  if (!akc && bkc) return launch_cfg<DT, 64, 64, false, true>(a, s);
-  return launch_cfg<DT, 64, 64, false, false>(a, s);
+  const dim3 g((unsigned)total), b(kThreads);
+  if (akc && bkc)
+    hipLaunchKernelGGL((gemm_unaligned_kernel<DT, true, true, T>), g, b, 0, s, a, vec_out);
+  else if (akc)
+    hipLaunchKernelGGL((gemm_unaligned_kernel<DT, true, false, T>), g, b, 0, s, a, vec_out);
+  else if (bkc)
+    hipLaunchKernelGGL((gemm_unaligned_kernel<DT, false, true, T>), g, b, 0, s, a, vec_out);
+  else
+    hipLaunchKernelGGL((gemm_unaligned_kernel<DT, false, false, T>), g, b, 0, s, a, vec_out);
+  return check_hip(hipGetLastError(), "gemm_unaligned launch");
 }
 
 bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
@@ -304,11 +267,20 @@ int32_t launch_gemm_mfma(const GemmProblem &p, hipStream_t s) {
   if (gemm_small_applicable(a, p.a_kcontig, p.b_kcontig))
     return launch_gemm_small(a, p.in_dt, p.a_kcontig, p.b_kcontig, s);
 
-  a.tiles_m = (int)((p.M + 63) / 64);
-  a.tiles_n = (int)((p.N + 63) / 64);
+  // 128 x 128 tiles when they fill the chip (two workgroups fit a CU), else
+  // 64 x 64.
+  const int cus = device_cu_count() > 0 ? device_cu_count() : 256;
+  const bool big = p.batch * ((p.M + 127) / 128) * ((p.N + 127) / 128) >= cus;
+  const int t = big ? 128 : 64;
+  a.tiles_m = (int)((p.M + t - 1) / t);
+  a.tiles_n = (int)((p.N + t - 1) / t);
+  const int w = a.out_dt == NOVA_HIP_DT_F32 ? 4 : 8;  // outputs per 16-byte store
+  const int vec_out = aligned16(a.C) && a.N % w == 0 && a.scm % w == 0 && a.scb % w == 0;
   if (p.in_dt == NOVA_HIP_DT_BF16)
-    return dispatch_layout<NOVA_HIP_DT_BF16>(a, p.a_kcontig, p.b_kcontig, s);
-  return dispatch_layout<NOVA_HIP_DT_F16>(a, p.a_kcontig, p.b_kcontig, s);
+    return big ? launch_cfg<NOVA_HIP_DT_BF16, 2>(a, vec_out, p.a_kcontig, p.b_kcontig, s)
+               : launch_cfg<NOVA_HIP_DT_BF16, 1>(a, vec_out, p.a_kcontig, p.b_kcontig, s);
+  return big ? launch_cfg<NOVA_HIP_DT_F16, 2>(a, vec_out, p.a_kcontig, p.b_kcontig, s)
+             : launch_cfg<NOVA_HIP_DT_F16, 1>(a, vec_out, p.a_kcontig, p.b_kcontig, s);
 }
 
 }  // namespace nova_hip
