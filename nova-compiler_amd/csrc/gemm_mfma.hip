@@ -192,7 +192,7 @@ __global__ __launch_bounds__(kThreads) void gemm_unaligned_kernel(GemmArgs a, in
     const int64_t at = (int64_t)bidx * a.scb + (int64_t)mb * a.scm + nw;
     if (a.out_dt == NOVA_HIP_DT_F32)
       ring::store_f32<32, 32 * T, 64, 1>(stg, 0, lane, static_cast<float *>(a.C) + at, a.scm,
-                                         a.M - mb, a.N - nw, vec_out, bias_w, has_gelu);
+                                         a.M - mb, a.N - nw, bias_w, has_gelu);
     else
       ring::store_16<32, 32 * T, 64, 1>(stg, 0, lane, static_cast<uint16_t *>(a.C) + at, a.scm,
                                         a.M - mb, a.N - nw, vec_out, bias_w, has_gelu,
@@ -274,8 +274,7 @@ int32_t launch_gemm_mfma(const GemmProblem &p, hipStream_t s) {
   const int t = big ? 128 : 64;
   a.tiles_m = (int)((p.M + t - 1) / t);
   a.tiles_n = (int)((p.N + t - 1) / t);
-  const int w = a.out_dt == NOVA_HIP_DT_F32 ? 4 : 8;  // outputs per 16-byte store
-  const int vec_out = aligned16(a.C) && a.N % w == 0 && a.scm % w == 0 && a.scb % w == 0;
+  const int vec_out = aligned16(a.C) && a.N % 8 == 0 && a.scm % 8 == 0 && a.scb % 8 == 0;
   if (p.in_dt == NOVA_HIP_DT_BF16)
     return big ? launch_cfg<NOVA_HIP_DT_BF16, 2>(a, vec_out, p.a_kcontig, p.b_kcontig, s)
                : launch_cfg<NOVA_HIP_DT_BF16, 1>(a, vec_out, p.a_kcontig, p.b_kcontig, s);

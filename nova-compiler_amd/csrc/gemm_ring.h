@@ -41,7 +41,7 @@ constexpr int BK = 64;
 
 struct RingArgs {
   GemmArgs g;
-  int vec_out;  // the output takes 16-byte stores (aligned rows of whole chunks)
+  int vec_out;  // a 16-bit output takes 16-byte stores (aligned rows of whole chunks)
 };
 
 // LDS chunk swizzles.  K-contiguous rows are those of gemm_dma.h.  A k-line
@@ -127,27 +127,29 @@ __device__ __forceinline__ uint16_t narrow(float x, bool bf16) {
   return bf16 ? to_bf16(x) : to_f16(x);
 }
 
+// 16 bytes at any 4-byte alignment.
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+
 // A staged ROWS x COLS block to C (its element (0, 0); `rows`, `cols` left
-// in the matrix) by NT threads, this one number tid.  16-byte stores: all of
-// a thread's chunks are read before the first is used.  Otherwise (rows not
-// 16-byte aligned) element stores, in a rolled loop, as is f32 output with
-// GELU (tanhf is large).
+// in the matrix) by NT threads, this one number tid.  All of a thread's
+// chunks are read before the first is used.  f32 rows need no alignment
+// beyond their own 4 bytes: 16-byte stores take any (element-by-element
+// stores of odd rows took 93.3 us where this takes 58.6 at 48x[997x64]x[64x997],
+// 59.5 against 50.6 at 4000x3002x1024; aligned rows the same either way).
+// f32 with GELU (tanhf is large) goes element by element in a rolled loop.
 template <int ROWS, int COLS, int NT, int KG>
 __device__ __forceinline__ void store_f32(char *stg, int dist, int tid, float *C, int64_t ld,
-                                          int rows, int cols, bool vec, const float *bias,
-                                          bool gelu) {
+                                          int rows, int cols, const float *bias, bool gelu) {
   constexpr int CR = COLS / 4, kIt = ROWS * CR / NT;  // 4-column chunks per row, per thread
   static_assert(ROWS * CR % NT == 0, "whole rounds");
-  if (gelu || !vec) {
+  if (gelu) {
 #pragma unroll 1
     for (int it = 0; it < kIt; ++it) {
       const int q = it * NT + tid, R = q / CR, c = q - R * CR;
       f32x4 x = staged_sum<COLS, KG>(stg, dist, R, c);
       if (bias) x = x + *reinterpret_cast<const f32x4 *>(bias + 4 * c);
-      if (gelu) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) x[e] = gelu_tanh(x[e]);
-      }
+      for (int e = 0; e < 4; ++e) x[e] = gelu_tanh(x[e]);
 #pragma unroll
       for (int e = 0; e < 4; ++e)
         if (R < rows && 4 * c + e < cols) C[R * ld + 4 * c + e] = x[e];
@@ -168,7 +170,13 @@ __device__ __forceinline__ void store_f32(char *stg, int dist, int tid, float *C
 #pragma unroll
   for (int it = 0; it < kIt; ++it) {
     const int q = it * NT + tid, R = q / CR, n = 4 * (q - R * CR);
-    if (R < rows && n < cols) *reinterpret_cast<f32x4 *>(C + R * ld + n) = x[it];
+    if (R < rows && n + 4 <= cols) {
+      *reinterpret_cast<f32x4u *>(C + R * ld + n) = x[it];
+    } else if (R < rows) {
+#pragma unroll
+      for (int e = 0; e < 3; ++e)
+        if (n + e < cols) C[R * ld + n + e] = x[it][e];
+    }
   }
 }
 
@@ -433,7 +441,7 @@ __global__ __launch_bounds__(kThreads * KG) void gemm_ring_kernel(RingArgs ra) {
       const int64_t at = (int64_t)bidx * a.scb + (int64_t)mb * a.scm + nw;
       if (a.out_dt == NOVA_HIP_DT_F32)
         store_f32<32, 32 * TN, 64, 1>(stg, 0, lane, static_cast<float *>(a.C) + at, a.scm, a.M - mb,
-                                      a.N - nw, ra.vec_out, bias_w, has_gelu);
+                                      a.N - nw, bias_w, has_gelu);
       else
         store_16<32, 32 * TN, 64, 1>(stg, 0, lane, static_cast<uint16_t *>(a.C) + at, a.scm,
                                      a.M - mb, a.N - nw, ra.vec_out, bias_w, has_gelu,
@@ -455,7 +463,7 @@ __global__ __launch_bounds__(kThreads * KG) void gemm_ring_kernel(RingArgs ra) {
     const float *bias_w = has_bias ? bias_s : nullptr;
     if (a.out_dt == NOVA_HIP_DT_F32)
       store_f32<BM, BN, kThreads * KG, KG>(smem, S * kStage, tid, static_cast<float *>(a.C) + at,
-                                           a.scm, a.M - m0, a.N - n0, ra.vec_out, bias_w, has_gelu);
+                                           a.scm, a.M - m0, a.N - n0, bias_w, has_gelu);
     else
       store_16<BM, BN, kThreads * KG, KG>(smem, S * kStage, tid, static_cast<uint16_t *>(a.C) + at,
                                           a.scm, a.M - m0, a.N - n0, ra.vec_out, bias_w, has_gelu,

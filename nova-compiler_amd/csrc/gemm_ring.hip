@@ -84,9 +84,8 @@ int32_t launch_gemm_aligned(const gemm::GemmArgs &a, int in_dt, bool akc, bool b
   r.g.tiles_m = (a.M + 64 * f.tm - 1) / (64 * f.tm);
   r.g.tiles_n = (a.N + 64 * f.tn - 1) / (64 * f.tn);
   r.g.round = cus % 8 == 0 ? cus * f.per_cu : 0;
-  const int w = a.out_dt == NOVA_HIP_DT_F32 ? 4 : 8;  // outputs per 16-byte store
-  r.vec_out = (reinterpret_cast<uintptr_t>(a.C) & 15u) == 0 && a.N % w == 0 && a.scm % w == 0 &&
-              a.scb % w == 0;
+  r.vec_out = (reinterpret_cast<uintptr_t>(a.C) & 15u) == 0 && a.N % 8 == 0 && a.scm % 8 == 0 &&
+              a.scb % 8 == 0;
   return in_dt == NOVA_HIP_DT_BF16 ? ring::launch_bf16(form, r, akc, bkc, s)
                                    : ring::launch_f16(form, r, akc, bkc, s);
 }
