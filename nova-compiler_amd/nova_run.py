@@ -85,6 +85,7 @@ class Program:
         self._p = lib().nova_run_parse(text.encode())
         if not self._p:
             _err("parse")
+        self._specs = {}  # per function: its arguments, its results
 
     def __del__(self):
         if getattr(self, "_p", None):
@@ -104,12 +105,24 @@ class Program:
         return dt.value, tuple(shape[d] for d in range(rank.value))
 
     def args(self, func: str):
+        spec = self._specs.get((func, "args"))
+        if spec is None:
+            spec = self._specs[func, "args"] = self._args(func)
+        return list(spec)
+
+    def results(self, func: str):
+        spec = self._specs.get((func, "results"))
+        if spec is None:
+            spec = self._specs[func, "results"] = self._results(func)
+        return list(spec)
+
+    def _args(self, func: str):
         n = lib().nova_run_num_args(self._p, func.encode())
         if n < 0:
             _err(f"@{func}")
         return [self._info(lib().nova_run_arg_info, func, i) for i in range(n)]
 
-    def results(self, func: str):
+    def _results(self, func: str):
         n = lib().nova_run_num_results(self._p, func.encode())
         if n < 0:
             _err(f"@{func}")

@@ -28,6 +28,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <atomic>
 #include <map>
 #include <memory>
 #include <mutex>
@@ -1229,15 +1230,26 @@ struct Planner {
         if (numel_of(src.shape) != numel_of(idx.shape) * base.shape[1])
           return fail(NOVA_HIP_ESHAPE, "line %d: nova.scatter_add src is not [indices, %lld]",
                       op.line, (long long)base.shape[1]);
-        // the op's result is a new tensor: the input copied, then the adds
-        View out = fresh(op.result_types[0]);
-        Step c;
-        c.kind = "copy";
-        c.in = {base};
-        c.out = {out};
-        c.text = "nova.scatter_add input -> hipMemcpyAsync(" + view_str(out) + " <- " +
-                 view_str(base) + ")";
-        plan.steps.push_back(c);
+        // the op's result is a new tensor: the input copied, then the adds;
+        // a splat constant that nothing else uses or names (a reshape of it,
+        // or it of another) is filled there to begin with
+        bool filled = false;
+        for (const Step &st : plan.steps)
+          for (const View &o : st.out)
+            if (o.buf == base.buf) filled = st.kind == "fill";
+        filled = filled && uses[op.operands[0]] == 1;
+        for (const auto &kv : env)
+          filled = filled && (kv.first == op.operands[0] || kv.second.buf != base.buf);
+        View out = filled ? base : fresh(op.result_types[0]);
+        if (!filled) {
+          Step c;
+          c.kind = "copy";
+          c.in = {base};
+          c.out = {out};
+          c.text = "nova.scatter_add input -> hipMemcpyAsync(" + view_str(out) + " <- " +
+                   view_str(base) + ")";
+          plan.steps.push_back(c);
+        }
         Step s;
         s.kind = "scatter";
         s.epi = idx.dt;
@@ -1720,7 +1732,12 @@ struct NovaRunProgram {
   // executions of one program never run on those buffers at once; and the
   // buffers are freed only once it has completed.
   mutable std::map<std::string, hipEvent_t> done;
-  int f32_gemm = NOVA_RUN_F32_GEMM_EXACT;  // nova_run_set_f32_gemm
+  std::atomic<int> f32_gemm{NOVA_RUN_F32_GEMM_EXACT};  // nova_run_set_f32_gemm
+  // Each function's plan per f32 GEMM mode: it depends on nothing else, and
+  // planning the GPT step took ~70 us, fifteen times per execution through
+  // the Python binding (its argument and result checks plan too).
+  mutable std::mutex plan_mu;
+  mutable std::map<std::pair<std::string, int>, std::shared_ptr<const Plan>> plans;
   const Func *find(const char *name) const {
     for (const Func &f : funcs)
       if (name && f.name == name) return &f;
@@ -1741,16 +1758,22 @@ struct NovaRunProgram {
 };
 
 namespace {
-int32_t plan_of(const NovaRunProgram *p, const char *func, Plan &out, const Func **fo) {
+int32_t plan_of(const NovaRunProgram *p, const char *func, std::shared_ptr<const Plan> &out,
+                const Func **fo) {
   t_err[0] = 0;
   if (!p) return fail(NOVA_HIP_EINVAL, "null program");
   const Func *f = p->find(func);
   if (!f) return fail(NOVA_HIP_EINVAL, "no function @%s", func ? func : "(null)");
-  Planner pl(*f, p->f32_gemm == NOVA_RUN_F32_GEMM_MFMA);
-  int32_t rc = pl.run();
-  if (rc) return rc;
-  out = pl.plan;
   if (fo) *fo = f;
+  const int mode = p->f32_gemm;
+  std::lock_guard<std::mutex> lock(p->plan_mu);
+  std::shared_ptr<const Plan> &held = p->plans[{f->name, mode}];
+  if (!held) {
+    Planner pl(*f, mode == NOVA_RUN_F32_GEMM_MFMA);
+    if (const int32_t rc = pl.run()) return rc;
+    held = std::make_shared<const Plan>(std::move(pl.plan));
+  }
+  out = held;
   return NOVA_HIP_SUCCESS;
 }
 
@@ -1824,9 +1847,9 @@ int32_t nova_run_num_args(const NovaRunProgram *p, const char *func) {
 }
 
 int32_t nova_run_num_results(const NovaRunProgram *p, const char *func) {
-  Plan pl;
+  std::shared_ptr<const Plan> pl;
   if (plan_of(p, func, pl, nullptr)) return -1;
-  return (int32_t)pl.results.size();
+  return (int32_t)pl->results.size();
 }
 
 int32_t nova_run_arg_info(const NovaRunProgram *p, const char *func, int32_t i, int32_t *dtype,
@@ -1839,9 +1862,10 @@ int32_t nova_run_arg_info(const NovaRunProgram *p, const char *func, int32_t i, 
 
 int32_t nova_run_result_info(const NovaRunProgram *p, const char *func, int32_t i,
                              int32_t *dtype, int32_t *rank, int64_t *shape) {
-  Plan pl;
-  int32_t rc = plan_of(p, func, pl, nullptr);
+  std::shared_ptr<const Plan> held;
+  int32_t rc = plan_of(p, func, held, nullptr);
   if (rc) return rc;
+  const Plan &pl = *held;
   if (i < 0 || i >= (int32_t)pl.results.size()) return fail(NOVA_HIP_EINVAL, "no result %d", i);
   const View &v = pl.results[i];
   fill_info(Type{v.shape, v.dt, false}, dtype, rank, shape);
@@ -1849,10 +1873,11 @@ int32_t nova_run_result_info(const NovaRunProgram *p, const char *func, int32_t 
 }
 
 int32_t nova_run_plan(const NovaRunProgram *p, const char *func, char *buf, size_t len) {
-  Plan pl;
+  std::shared_ptr<const Plan> plan;
   const Func *f = nullptr;
-  int32_t rc = plan_of(p, func, pl, &f);
+  int32_t rc = plan_of(p, func, plan, &f);
   if (rc) return rc;
+  const Plan &pl = *plan;
   std::string s = "func @" + f->name + ":\n";
   for (const Step &st : pl.steps) s += "  " + st.text + "\n";
   s += "  return";
@@ -1867,10 +1892,11 @@ int32_t nova_run_plan(const NovaRunProgram *p, const char *func, char *buf, size
 
 int32_t nova_run_execute(const NovaRunProgram *p, const char *func, const void *const *host_args,
                          void *const *host_results) {
-  Plan pl;
+  std::shared_ptr<const Plan> plan;
   const Func *f = nullptr;
-  int32_t rc = plan_of(p, func, pl, &f);
+  int32_t rc = plan_of(p, func, plan, &f);
   if (rc) return rc;
+  const Plan &pl = *plan;
   if ((!host_args && !f->arg_types.empty()) || (!host_results && !pl.results.empty()))
     return fail(NOVA_HIP_EINVAL, "null argument or result array");
   hipStream_t st = static_cast<hipStream_t>(nova_hip_get_stream());
@@ -1947,10 +1973,11 @@ int32_t nova_run_execute(const NovaRunProgram *p, const char *func, const void *
 
 int32_t nova_run_execute_device(const NovaRunProgram *p, const char *func,
                                 void *const *dev_args, void *const *dev_results) {
-  Plan pl;
+  std::shared_ptr<const Plan> plan;
   const Func *f = nullptr;
-  int32_t rc = plan_of(p, func, pl, &f);
+  int32_t rc = plan_of(p, func, plan, &f);
   if (rc) return rc;
+  const Plan &pl = *plan;
   if ((!dev_args && !f->arg_types.empty()) || (!dev_results && !pl.results.empty()))
     return fail(NOVA_HIP_EINVAL, "null argument or result array");
   for (size_t i = 0; i < f->arg_types.size(); ++i)
