@@ -85,7 +85,7 @@ int32_t nova_run_execute_device(const NovaRunProgram *p, const char *func,
 /* How f32 GEMMs (nova.matmul / nova.linear / linalg.matmul on f32 and their
  * backward ops) are planned.  EXACT (the default): sequential k with
  * separately rounded multiply and add, bit-identical to Nova's CPU pipeline
- * (Pipeline.cpp:61-187).  MFMA: the f32 matrix cores
+ * (Pipeline.cpp:61-187).  MFMA: f32 on the matrix cores
  * (NOVA_HIP_GEMM_F32_MFMA of nova_hip.h), within the f32 parity bar (1e-4
  * relative) but not bit-identical, several times faster. */
 enum { NOVA_RUN_F32_GEMM_EXACT = 0, NOVA_RUN_F32_GEMM_MFMA = 1 };

@@ -1,6 +1,6 @@
 // The LDS-DMA pieces shared by the MFMA GEMMs of 16-byte aligned operands:
-// the persistent 256x256 kernel (gemm_pers.h: whole tiles, at least one full
-// round of them) and the ring kernel (gemm_ring.h: every other shape).
+// the persistent 256x256 kernel (gemm_pers.h: whole tiles) and the ring
+// kernel (gemm_ring.h: any shape).
 //
 // Operands travel global -> LDS with buffer_load ... lds (LDS DMA): no
 // staging registers.  K is consumed in steps of BK = 64 so that every

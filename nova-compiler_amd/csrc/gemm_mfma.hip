@@ -6,8 +6,8 @@
 // 115-372: tile+distribute, pad, promote to shared memory, mma.sync,
 // 3-stage cp.async).  The kernels, chosen per problem by launch_gemm_mfma:
 //
-//  * operands with 16-byte aligned rows: gemm_pers.h (whole 256x256 tiles,
-//    at least a round of them) and gemm_ring.h (every other shape);
+//  * operands with 16-byte aligned rows: gemm_pers.h (whole 256x256 tiles)
+//    or gemm_ring.h (any shape), by estimated time;
 //  * unaligned rows: gemm_small.hip when the whole K of a tile fits LDS, else
 //    the kernel in this file.
 //

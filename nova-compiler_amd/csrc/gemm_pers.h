@@ -6,8 +6,7 @@
 //
 // Workgroup g of G takes tiles g, g + G, g + 2G, ... in round_tile_of
 // order (G = a.round, one per CU), i.e. the same tile -> CU assignment as
-// the one-tile-per-workgroup kernel.  The K loop, LDS ring and swizzles are
-// those of gemm_dma_kernel.  Differences:
+// one workgroup per tile.  Beside the ring and swizzles of gemm_dma.h:
 //   * each DMA offset is a lane part (fixed) plus a wave-uniform tile and
 //     K part, so the loads can target the next tile;
 //   * the last K step of a tile issues all of the next tile's second K step
@@ -29,7 +28,7 @@ using namespace gemm;
 using namespace dma;
 
 // Tile-independent part of each DMA byte offset of this lane: load i of
-// wave w fills slots [(i*4 + w) * 64, +64) of a stage, as in dma_setup.
+// wave w fills slots [(i*4 + w) * 64, +64) of a stage.
 template <bool KC>
 __device__ __forceinline__ void lane_offsets(uint32_t (&off)[kLoads], int64_t s_outer, int wave,
                                              int lane) {
@@ -242,7 +241,7 @@ __global__ __launch_bounds__(kThreads) void gemm_pers_kernel(GemmArgs a) {
   __builtin_amdgcn_sched_barrier(0);
 
   int cur = 0;
-  // K step kt of the current tile, as in gemm_dma_kernel.  KIND 0: the
+  // K step kt of the current tile.  KIND 0: the
   // tile's first, whose successor was issued whole before (after an
   // epilogue, ahead of its stores); 1: a middle one; 2: the last, which
   // issues all of the next tile's second K step (the next tile's first

@@ -5,7 +5,7 @@
 // K shared by several groups of waves where a shape has few tiles.
 //
 // What bounds it: large tiles by MFMA issue and the board's power limit, as
-// gemm_dma_kernel; small ones by the latency of the DMA a stage ahead, which
+// gemm_pers.h; small ones by the latency of the DMA a stage ahead, which
 // is why the small tiles have more stages and several workgroups per CU.
 //
 // Four wave64s in a 2 x 2 grid own (32 TM) x (32 TN) outputs each, so the

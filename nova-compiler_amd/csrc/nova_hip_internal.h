@@ -53,7 +53,7 @@ int32_t launch_gemm_mfma(const GemmProblem &p, hipStream_t s);
 // Launch the exact kernel: f32 in and out, or (acc_out) bf16 / f16 in and
 // out with the accumulator in that type.
 int32_t launch_gemm_exact(const GemmProblem &p, hipStream_t s);
-// f32 in and out on the f32 MFMA (NOVA_HIP_GEMM_F32_MFMA): within the f32
+// f32 in and out on the matrix cores (NOVA_HIP_GEMM_F32_MFMA): within the f32
 // parity bar, not bit-identical to the sequential-k reference arithmetic.
 int32_t launch_gemm_f32_mfma(const GemmProblem &p, hipStream_t s);
 

@@ -232,7 +232,7 @@ def gemm(A, B, out=None, *, bias=None, epilogue: int = EPI_NONE, out_dtype=None,
     transposed views included); returns C [Bt,M,N] (or [M,N] for rank-2
     inputs) in ``out_dtype`` (f32 by default).  ``acc_out``: accumulate in
     the output dtype (NOVA_HIP_GEMM_ACC_OUT; bf16 / f16 in and out).
-    ``f32_mfma``: f32 operands on the f32 matrix cores (NOVA_HIP_GEMM_F32_MFMA;
+    ``f32_mfma``: f32 operands on the matrix cores (NOVA_HIP_GEMM_F32_MFMA;
     within 1e-4, not bit-identical to the sequential-k reference).
     ``acc_c``: ``out`` holds the accumulators' initial values and receives
     out + A . B in place (NOVA_HIP_GEMM_ACC_C, linalg.matmul on data-holding

@@ -136,7 +136,7 @@ class Program:
 
     def set_f32_gemm(self, mode: int) -> None:
         """F32_GEMM_EXACT (bit-identical to the reference's CPU arithmetic) or
-        F32_GEMM_MFMA (the f32 matrix cores, within 1e-4)."""
+        F32_GEMM_MFMA (f32 on the matrix cores, within 1e-4)."""
         if lib().nova_run_set_f32_gemm(self._p, mode):
             _err("set_f32_gemm")
 
