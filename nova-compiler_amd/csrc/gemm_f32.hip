@@ -421,26 +421,31 @@ __global__ __launch_bounds__(256) void gemm_exact_vec_kernel(F32Args a, uint32_t
 
 // The tiny form, for problems whose vector-form tiles leave CUs idle (config
 // 1, 256^3: the 64x32 form's 32 tiles occupy 32 of 256 CUs, each thread
-// running eight 256-long chains): a 16x16 tile per 256-thread workgroup,
-// one output per thread.  Per stage of KS k each thread loads KS / 64 float4
-// of A and of B along their unit-stride dims; LDS holds A as [m][k] and B
+// running eight 256-long chains): a 16x16 tile per workgroup of 256 / RM
+// threads, RM outputs of one column per thread.  Per stage of KS k each thread
+// loads RM KS / 64 float4 of A and of B along their unit-stride dims; LDS holds A as [m][k] and B
 // as [n][k] (KS + 4 floats apart: the 16 columns a wave reads fall on 64
-// distinct banks), so a thread reads four k of its row and of its column
-// with two 16-byte reads.  The arithmetic per output is the other forms'.
+// distinct banks), so a thread reads four k of its rows and of its column
+// with 1 + RM 16-byte reads, those of the next four k in flight while it
+// multiplies (us without that and with: 512 x 384 x 50304 790 -> 752,
+// 64 x 64 x 1024 12.2 -> 10.2, 256^3 5.2 -> 4.6 through the Python binding;
+// four groups ahead gain another 4% at 256^3 and lose 4% at 512 x 384 x 50304).
+// RM = 2 reads a quarter less LDS per output, at half the waves.  The arithmetic per output is the other forms'.
 // Stages of 128 k (in-process A/B, us, stages of 64 / 128 / 256): 256^3
 // 4.88 / 4.75 / 4.50, 512^3 12.84 / 12.42 / 13.95 (256-deep stages leave
 // two workgroups per CU), 64x64x1024 13.4 / 12.1 / 11.2; the 64x32 form
 // took 14.1, 25.7 and 47.9.
 constexpr int kTinyKs = 128;
 
-template <bool AKC, bool BKC>
-__global__ __launch_bounds__(256) void gemm_exact_tiny_kernel(F32Args a, uint32_t a_bytes,
-                                                               uint32_t b_bytes) {
+template <bool AKC, bool BKC, int RM>
+__global__ __launch_bounds__(256 / RM) void gemm_exact_tiny_kernel(F32Args a, uint32_t a_bytes,
+                                                                   uint32_t b_bytes) {
 #pragma clang fp contract(off)
   typedef float f32x4 __attribute__((ext_vector_type(4)));
   constexpr int KS = kTinyKs, P = KS + 4;
-  constexpr int E = KS / 64;  // float4 of each operand per thread per stage
-  static_assert(KS % 64 == 0, "a stage is a whole number of float4 per thread");
+  constexpr int NT = 256 / RM, TY = kVt / RM;
+  constexpr int E = 4 * KS / NT;  // float4 of each operand per thread per stage
+  static_assert(4 * KS % NT == 0, "a stage is a whole number of float4 per thread");
   __shared__ __attribute__((aligned(16))) float sa[2][kVt * P];
   __shared__ __attribute__((aligned(16))) float sb[2][kVt * P];
   const int tiles = a.tiles_m * a.tiles_n;
@@ -452,7 +457,7 @@ __global__ __launch_bounds__(256) void gemm_exact_tiny_kernel(F32Args a, uint32_
   const int64_t sb_outer = BKC ? a.sbn : a.sbk;
   const __amdgpu_buffer_rsrc_t ra = f32_rsrc(static_cast<const float *>(a.A) + b * a.sab, a_bytes);
   const __amdgpu_buffer_rsrc_t rb = f32_rsrc(static_cast<const float *>(a.B) + b * a.sbb, b_bytes);
-  // float4 q = tid + 256 e of a stage: K-contiguous, row q / (KS / 4) and
+  // float4 q = tid + NT e of a stage: K-contiguous, row q / (KS / 4) and
   // k 4 (q % (KS / 4)); otherwise k q / 4 and rows 4 (q % 4) .. + 3.  Rows
   // past M / N read neighbouring data or zero (their outputs are not
   // stored); k past K is never multiplied.
@@ -466,7 +471,7 @@ __global__ __launch_bounds__(256) void gemm_exact_tiny_kernel(F32Args a, uint32_
   auto gload = [&](int k0) __attribute__((always_inline)) {
 #pragma unroll
     for (int e = 0; e < E; ++e) {
-      const int q = tid + 256 * e;
+      const int q = tid + NT * e;
       ga[e] = ld4(ra, AKC ? (int64_t)(m0 + row_of(q)) * sa_outer + k0 + k4_of(q)
                           : (int64_t)(k0 + q / 4) * sa_outer + m0 + (q % 4) * 4);
       gb[e] = ld4(rb, BKC ? (int64_t)(n0 + row_of(q)) * sb_outer + k0 + k4_of(q)
@@ -476,7 +481,7 @@ __global__ __launch_bounds__(256) void gemm_exact_tiny_kernel(F32Args a, uint32_
   auto sstore = [&](int buf) __attribute__((always_inline)) {
 #pragma unroll
     for (int e = 0; e < E; ++e) {
-      const int q = tid + 256 * e;
+      const int q = tid + NT * e;
       if (AKC) {
         *reinterpret_cast<f32x4 *>(&sa[buf][row_of(q) * P + k4_of(q)]) = ga[e];
       } else {
@@ -491,13 +496,19 @@ __global__ __launch_bounds__(256) void gemm_exact_tiny_kernel(F32Args a, uint32_
       }
     }
   };
-  const int m = m0 + ty, n = n0 + tx;
   const bool has_bias = (a.epi == NOVA_HIP_EPI_BIAS || a.epi == NOVA_HIP_EPI_BIAS_GELU);
   const bool has_gelu = (a.epi == NOVA_HIP_EPI_BIAS_GELU || a.epi == NOVA_HIP_EPI_GELU);
-  float acc = (has_bias && n < a.N) ? bias_value(a.bias, a.bias_dt, n) : 0.0f;
-  // linalg.matmul on data-holding outs: the sum starts from C's value.
-  if (a.acc_c && m < a.M && n < a.N)
-    acc = static_cast<const float *>(a.C)[(int64_t)b * a.scb + (int64_t)m * a.scm + n];
+  // Output i of this thread: row m0 + ty + i TY.
+  const int n = n0 + tx;
+  float acc[RM];
+#pragma unroll
+  for (int i = 0; i < RM; ++i) {
+    const int m = m0 + ty + i * TY;
+    acc[i] = (has_bias && n < a.N) ? bias_value(a.bias, a.bias_dt, n) : 0.0f;
+    // linalg.matmul on data-holding outs: the sum starts from C's value.
+    if (a.acc_c && m < a.M && n < a.N)
+      acc[i] = static_cast<const float *>(a.C)[(int64_t)b * a.scb + (int64_t)m * a.scm + n];
+  }
   gload(0);
   sstore(0);
   __syncthreads();
@@ -507,30 +518,46 @@ __global__ __launch_bounds__(256) void gemm_exact_tiny_kernel(F32Args a, uint32_
     if (more) gload(k0 + KS);
     const float *ar = &sa[buf][ty * P], *br = &sb[buf][tx * P];
     if (a.K - k0 >= KS) {
-#pragma unroll 4
-      for (int kq = 0; kq < KS / 4; ++kq) {
-        const f32x4 av = *reinterpret_cast<const f32x4 *>(ar + 4 * kq);
-        const f32x4 bv = *reinterpret_cast<const f32x4 *>(br + 4 * kq);
+      f32x4 av[2][RM], bv[2];
+      auto read = [&](int set, int kq) __attribute__((always_inline)) {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const float p = av[u] * bv[u];
-          acc = acc + p;
-        }
+        for (int i = 0; i < RM; ++i)
+          av[set][i] = *reinterpret_cast<const f32x4 *>(ar + i * TY * P + 4 * kq);
+        bv[set] = *reinterpret_cast<const f32x4 *>(br + 4 * kq);
+      };
+      read(0, 0);
+#pragma unroll
+      for (int kq = 0; kq < KS / 4; ++kq) {
+        if (kq + 1 < KS / 4) read((kq + 1) & 1, kq + 1);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+          for (int i = 0; i < RM; ++i) {
+            const float p = av[kq & 1][i][u] * bv[kq & 1][u];
+            acc[i] = acc[i] + p;
+          }
+        __builtin_amdgcn_sched_barrier(0);
       }
     } else {
       // The last, partial stage: only its real k (a padded k would add
       // 0 * b, which turns a -0 sum into +0 and an infinite b into NaN).
-      for (int kk = 0; kk < a.K - k0; ++kk) {
-        const float p = ar[kk] * br[kk];
-        acc = acc + p;
-      }
+      for (int kk = 0; kk < a.K - k0; ++kk)
+#pragma unroll
+        for (int i = 0; i < RM; ++i) {
+          const float p = ar[i * TY * P + kk] * br[kk];
+          acc[i] = acc[i] + p;
+        }
     }
     if (more) sstore(buf ^ 1);
     __syncthreads();
     buf ^= 1;
   }
-  if (m < a.M && n < a.N) {
-    float v = acc;
+#pragma unroll
+  for (int i = 0; i < RM; ++i) {
+    const int m = m0 + ty + i * TY;
+    if (m >= a.M || n >= a.N) continue;
+    float v = acc[i];
     if (has_gelu) v = gelu_ref(v);
     static_cast<float *>(a.C)[(int64_t)b * a.scb + (int64_t)m * a.scm + n] = v;
   }
@@ -550,17 +577,18 @@ constexpr VecForm kVecForms[] = {{8, 8, 16, 1.0}, {4, 8, 16, 0.95}, {4, 6, 32, 0
 constexpr int kNumVecForms = sizeof(kVecForms) / sizeof(kVecForms[0]);
 constexpr double kTinyRate = 0.5;
 
-template <bool AKC, bool BKC>
-void launch_tiny_t(const F32Args &a, uint32_t ab, uint32_t bb, unsigned grid, hipStream_t s) {
-  hipLaunchKernelGGL((gemm_exact_tiny_kernel<AKC, BKC>), dim3(grid), dim3(256), 0, s, a, ab, bb);
-}
-
+template <int RM>
 void launch_tiny(const F32Args &a, bool akc, bool bkc, uint32_t ab, uint32_t bb, unsigned grid,
                  hipStream_t s) {
-  if (akc && bkc) launch_tiny_t<true, true>(a, ab, bb, grid, s);
-  else if (akc) launch_tiny_t<true, false>(a, ab, bb, grid, s);
-  else if (bkc) launch_tiny_t<false, true>(a, ab, bb, grid, s);
-  else launch_tiny_t<false, false>(a, ab, bb, grid, s);
+  const dim3 g(grid), blk(256 / RM);
+  if (akc && bkc)
+    hipLaunchKernelGGL((gemm_exact_tiny_kernel<true, true, RM>), g, blk, 0, s, a, ab, bb);
+  else if (akc)
+    hipLaunchKernelGGL((gemm_exact_tiny_kernel<true, false, RM>), g, blk, 0, s, a, ab, bb);
+  else if (bkc)
+    hipLaunchKernelGGL((gemm_exact_tiny_kernel<false, true, RM>), g, blk, 0, s, a, ab, bb);
+  else
+    hipLaunchKernelGGL((gemm_exact_tiny_kernel<false, false, RM>), g, blk, 0, s, a, ab, bb);
 }
 
 template <int RM, int CN, int KS>
@@ -654,8 +682,13 @@ int32_t launch_gemm_exact(const GemmProblem &p, hipStream_t s) {
         if ((double)waves * (kVt * kVt) / kTinyRate < best_cost) {
           a.tiles_m = (int)((p.M + kVt - 1) / kVt);
           a.tiles_n = (int)((p.N + kVt - 1) / kVt);
-          launch_tiny(a, p.a_kcontig, p.b_kcontig, (uint32_t)(a_ext * 4), (uint32_t)(b_ext * 4),
-                      (unsigned)tiny_tiles, s);
+          // Two outputs per thread from three tiles per CU on, where LDS
+          // bandwidth bounds it; one below, where each CU's few waves do
+          // (512 x 384 x 50304, 3 tiles: 680 us against 752; 512^3, 4:
+          // 10.2 / 11.8; 320 x 320 x 1024, 1.6: 15.5 / 12.4; 256^3, 1: 5.8 / 4.6).
+          auto *launch = tiny_tiles > 2 * (int64_t)cus ? launch_tiny<2> : launch_tiny<1>;
+          launch(a, p.a_kcontig, p.b_kcontig, (uint32_t)(a_ext * 4), (uint32_t)(b_ext * 4),
+                 (unsigned)tiny_tiles, s);
           return check_hip(hipGetLastError(), "gemm_exact launch");
         }
       }
