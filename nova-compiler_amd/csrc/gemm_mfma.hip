@@ -36,9 +36,11 @@ struct Chunk {
   uint32_t hi;
 };
 
+// The 16 goes into the address (the instruction's own offset, which the range
+// check counts), not into the scalar offset operand, which it need not.
 __device__ __forceinline__ Chunk load_chunk(__amdgpu_buffer_rsrc_t r, uint32_t off) {
   return Chunk{__builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0),
-               (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(r, off, 16, 0)};
+               (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(r, off + 16u, 0, 0)};
 }
 
 // The chunk's eight elements, with only the first `left` kept.

@@ -61,3 +61,17 @@ def test_unaligned_epilogues(cuda, epi, out):
         ref = torch.nn.functional.gelu(ref, approximate="tanh")
     tol = 2e-6 * (1 + ref.abs()) if out == "f32" else 2.0 ** -8 * ref.abs() + 1e-6
     assert bool(((got - ref).abs() <= tol).all())
+
+
+@pytest.mark.parametrize("M,N", [(3, 65), (130, 5), (1, 2)])
+def test_unaligned_operand_slices_shorter_than_a_chunk(cuda, M, N):
+    """Operands whose K stride is zero: the whole slice is one line of M (or N)
+    elements, down to two bytes."""
+    import torch
+    K = 577
+    g = torch.Generator().manual_seed(M)
+    for dt in (torch.bfloat16, torch.float16):
+        a = torch.randint(-4, 5, (M,), generator=g).to(cuda).to(dt)
+        b = torch.randint(-4, 5, (N,), generator=g).to(cuda).to(dt)
+        C = nh.gemm(a.as_strided((1, M, K), (0, 1, 0)), b.as_strided((1, K, N), (0, 0, 1)))
+        assert torch.equal(C[0].double(), K * torch.outer(a.double(), b.double())), dt
