@@ -124,17 +124,30 @@ __device__ __forceinline__ Pieces split8(Raw r, uint32_t sign) {
 // XOR of a chunk index of k-line k of an M/N-contiguous stage.
 __device__ __forceinline__ int line_swz(int k) { return (k & 8); }
 
-// Byte offset from the operand's stage base of this lane's first read of a
-// fragment (rows row_base + lane % 32, k = 16 kk + 8 (lane / 32) ... + 7).
+// Fragment f of a wave (rows row_base + 32 f + lane % 32, k = 16 kk + 8
+// (lane / 32) ... + 7) is read at frag_base of parity frag_parity(f, kk),
+// frag_fixed bytes on: 32 rows on, a K-contiguous row's swizzle has its bit 2
+// changed, as it has at the other kk, and the swizzle of an M/N-contiguous
+// line turns the step of 8 chunks round in the lanes of one half.  Two
+// registers per operand hold all of a wave's offsets.
 template <bool KC, int R>
-__device__ __forceinline__ uint32_t frag_offset(int row_base, int kk, int lane) {
-  const int row = row_base + (lane & 31), h = lane >> 5;
+__device__ __forceinline__ uint32_t frag_base(int row_base, int parity, int lane) {
+  const int h = lane >> 5;
   if constexpr (KC) {
-    return (uint32_t)(row * 8 + ((kk * 4 + h * 2) ^ ((row ^ (row >> 3)) & 7))) * 16u;
+    const int row = row_base + (lane & 31);
+    return (uint32_t)(row * 8 + ((parity * 4 + h * 2) ^ ((row ^ (row >> 3)) & 7))) * 16u;
   } else {
-    const int k = kk * 16 + h * 8;
+    const int row = row_base + 32 * parity + (lane & 31), k = h * 8;
     return (uint32_t)(k * R + ((((row >> 2) ^ line_swz(k)) << 2) | (row & 3))) * 4u;
   }
+}
+template <bool KC>
+constexpr int frag_parity(int f, int kk) {
+  return KC ? (f ^ kk) & 1 : f & 1;
+}
+template <bool KC, int R>
+constexpr int frag_fixed(int f, int kk) {
+  return KC ? f * 32 * 128 : (f >> 1) * 64 * 4 + kk * 16 * R * 4;
 }
 
 typedef float f32x2 __attribute__((ext_vector_type(2)));
@@ -144,16 +157,26 @@ __device__ __forceinline__ f32x2 lds_read2st64(uint32_t addr) {
   asm volatile("ds_read2st64_b32 %0, %1 offset0:%2 offset1:%3" : "=v"(v) : "v"(addr), "n"(O0), "n"(O1));
   return v;
 }
-template <bool KC, int R>
+template <int O>
+__device__ __forceinline__ f32x4 lds_read_b128_at(uint32_t addr) {
+  f32x4 v;
+  asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(O));
+  return v;
+}
+// The fragment O bytes past addr.
+template <bool KC, int R, int O>
 __device__ __forceinline__ Raw read_raw(uint32_t addr) {
   Raw r;
   if constexpr (KC) {
-    r.v[0] = __builtin_bit_cast(f32x4, dma::lds_read_b128(addr));
-    r.v[1] = __builtin_bit_cast(f32x4, dma::lds_read_b128(addr ^ 16u));
+    static_assert(O < 65536, "offset range");
+    r.v[0] = lds_read_b128_at<O>(addr);
+    r.v[1] = lds_read_b128_at<O>(addr ^ 16u);
   } else {
-    constexpr int P = R / 64;  // a k-line in units of 64 dwords
-    const f32x2 a = lds_read2st64<0, P>(addr), b = lds_read2st64<2 * P, 3 * P>(addr);
-    const f32x2 c = lds_read2st64<4 * P, 5 * P>(addr), d = lds_read2st64<6 * P, 7 * P>(addr);
+    constexpr int P = R / 64, Q = O / 256;  // a k-line, the offset in units of 64 dwords
+    static_assert(O % 256 == 0 && Q + 7 * P < 256, "offset range");
+    const f32x2 a = lds_read2st64<Q, Q + P>(addr), b = lds_read2st64<Q + 2 * P, Q + 3 * P>(addr);
+    const f32x2 c = lds_read2st64<Q + 4 * P, Q + 5 * P>(addr);
+    const f32x2 d = lds_read2st64<Q + 6 * P, Q + 7 * P>(addr);
     r.v[0] = f32x4{a[0], a[1], b[0], b[1]};
     r.v[1] = f32x4{c[0], c[1], d[0], d[1]};
   }
@@ -272,7 +295,10 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_split_kernel(SplitArgs a) {
   const int units = (total - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x * a.chunks;
 
   // As in gemm_ring.h: byte offset (at k = 0, from the tile's first row) and
-  // k within a K step of the chunk this lane's DMA load i fetches.
+  // k within a K step of the chunk this lane's DMA load i fetches.  The
+  // pattern repeats after 64 rows (two loads) of a K-contiguous operand and
+  // after 16 k-lines (TM or TN loads) of the other: a lane keeps one period,
+  // and what later loads add is the same for all lanes.
   auto setup = [&](auto kc, auto rows, int64_t s_outer, int i, uint32_t &off, int &kl)
                    __attribute__((always_inline)) {
     constexpr bool KC = decltype(kc)::value;
@@ -288,14 +314,15 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_split_kernel(SplitArgs a) {
       off = (uint32_t)(((int64_t)k * s_outer + c * 4) * 4);
     }
   };
-  uint32_t oa[LA], ob[LB];
-  int ka[LA], kb[LB];
+  constexpr int PA = AKC ? 2 : TM, PB = BKC ? 2 : TN;
+  uint32_t oa[PA], ob[PB];
+  int ka[PA], kb[PB];
 #pragma unroll
-  for (int i = 0; i < LA; ++i)
+  for (int i = 0; i < PA; ++i)
     setup(std::integral_constant<bool, AKC>{}, std::integral_constant<int, BM>{}, a.sa_outer, i,
           oa[i], ka[i]);
 #pragma unroll
-  for (int i = 0; i < LB; ++i)
+  for (int i = 0; i < PB; ++i)
     setup(std::integral_constant<bool, BKC>{}, std::integral_constant<int, BN>{}, a.sb_outer, i,
           ob[i], kb[i]);
   // The next K step to fetch: S steps ahead of the one being multiplied.
@@ -307,8 +334,9 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_split_kernel(SplitArgs a) {
     int unit;
     Tile t;
   } next;
-  const uint32_t step_a = AKC ? BK * 4u : (uint32_t)(BK * a.sa_outer * 4);
-  const uint32_t step_b = BKC ? BK * 4u : (uint32_t)(BK * a.sb_outer * 4);
+  const uint32_t row_a = (uint32_t)(a.sa_outer * 4), row_b = (uint32_t)(a.sb_outer * 4);
+  const uint32_t step_a = AKC ? BK * 4u : BK * row_a;
+  const uint32_t step_b = BKC ? BK * 4u : BK * row_b;
   auto next_unit = [&](int u) __attribute__((always_inline)) {
     next.unit = u;
     next.left = next.steps = 0;
@@ -332,12 +360,17 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_split_kernel(SplitArgs a) {
   // read for k >= K.
   auto dma = [&](int q, int st) __attribute__((always_inline)) {
     char *base = smem + st * kStage;
-    if (q < LA)
+    if (q < LA) {
+      const int p = q / PA;
+      const uint32_t at = next.at_a + (uint32_t)(p * (AKC ? 64 : 16)) * row_a;
       dma16(next.A, a.a_bytes, base + (q * 4 + wave) * 1024,
-            ka[q] < next.left ? oa[q] + next.at_a : kOOB);
-    else
-      dma16(next.B, a.b_bytes, base + kStageA + ((q - LA) * 4 + wave) * 1024,
-            kb[q - LA] < next.left ? ob[q - LA] + next.at_b : kOOB);
+            ka[q % PA] < next.left - (AKC ? 0 : 16 * p) ? oa[q % PA] + at : kOOB);
+    } else {
+      const int r = q - LA, p = r / PB;
+      const uint32_t at = next.at_b + (uint32_t)(p * (BKC ? 64 : 16)) * row_b;
+      dma16(next.B, a.b_bytes, base + kStageA + (r * 4 + wave) * 1024,
+            kb[r % PB] < next.left - (BKC ? 0 : 16 * p) ? ob[r % PB] + at : kOOB);
+    }
   };
   // With K not a multiple of 4, the last chunk of a K-contiguous row holds
   // values of the next row: zero them once the K step holding it has landed.
@@ -353,16 +386,21 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_split_kernel(SplitArgs a) {
     __syncthreads();
   };
 
-  uint32_t fofs[2][F];
+  uint32_t fofs_a[2], fofs_b[2];
 #pragma unroll
-  for (int kk = 0; kk < 2; ++kk)
-#pragma unroll
-    for (int f = 0; f < F; ++f)
-      fofs[kk][f] = f < TM ? frag_offset<AKC, BM>(am + f * 32, kk, lane)
-                           : kStageA + frag_offset<BKC, BN>(bn + (f - TM) * 32, kk, lane);
+  for (int p = 0; p < 2; ++p) {
+    fofs_a[p] = frag_base<AKC, BM>(am, p, lane);
+    fofs_b[p] = kStageA + frag_base<BKC, BN>(bn, p, lane);
+  }
   const uint32_t lds0 = lds_addr(smem);
-  auto read_one = [&](int f, uint32_t stage, int kk) __attribute__((always_inline)) {
-    return f < TM ? read_raw<AKC, BM>(stage + fofs[kk][f]) : read_raw<BKC, BN>(stage + fofs[kk][f]);
+  // Fragment f (A's first, then B's) of k16 step kk of the stage at `stage`.
+  auto read_one = [&](auto fc, uint32_t stage, auto kkc) __attribute__((always_inline)) {
+    constexpr int f = decltype(fc)::value, kk = decltype(kkc)::value;
+    if constexpr (f < TM)
+      return read_raw<AKC, BM, frag_fixed<AKC, BM>(f, kk)>(stage + fofs_a[frag_parity<AKC>(f, kk)]);
+    else
+      return read_raw<BKC, BN, frag_fixed<BKC, BN>(f - TM, kk)>(
+          stage + fofs_b[frag_parity<BKC>(f - TM, kk)]);
   };
 
   f32x16 acc[TM][TN];
@@ -382,15 +420,14 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_split_kernel(SplitArgs a) {
   NOVA_WAIT_VMCNT((S - 1) * L);
   __builtin_amdgcn_s_barrier();
   if (tail && tc.kt0 == last_kt) zero_tail(0);
-#pragma unroll
-  for (int f = 0; f < F; ++f) {
+  static_for<F>([&](auto f) __attribute__((always_inline)) {
     __builtin_amdgcn_sched_barrier(0);
-    const Raw r = read_one(f, lds0, 0);
+    const Raw r = read_one(f, lds0, std::integral_constant<int, 0>{});
     NOVA_WAIT_LGKMCNT0();
     __builtin_amdgcn_sched_barrier(0);
-    if (f < TM) pa[0][f] = split8<!kFlipB>(r, tc.sign);
+    if constexpr (f < TM) pa[0][f] = split8<!kFlipB>(r, tc.sign);
     else pb[f - TM] = split8<kFlipB>(r, tc.sign);
-  }
+  });
 
   // One k16 step with A's pieces in pa[KK]: the MFMAs of column block j are
   // phase j, the six partial products of each of its TM tiles, the smallest
@@ -407,7 +444,8 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_split_kernel(SplitArgs a) {
       __builtin_amdgcn_sched_barrier(0);
       Raw raw[NF];
       static_for<NF>([&](auto n) __attribute__((always_inline)) {
-        raw[n] = read_one(phase_frag<TM, TN>(j, n), from, KK ^ 1);
+        raw[n] = read_one(std::integral_constant<int, phase_frag<TM, TN>(j, n)>{}, from,
+                          std::integral_constant<int, KK ^ 1>{});
       });
       if constexpr (KK == 1) {
         constexpr int kPer = (L + TN - 1) / TN;

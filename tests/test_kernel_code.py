@@ -52,3 +52,51 @@ def test_gemm_loads_are_inside_the_range_check(objects):
                 seen += 1
                 assert re.search(r"s\[\d+:\d+\], 0( |$)", i), (name, i)
     assert seen > 100
+
+
+def _registers(text):
+    """The vector registers an operand list names, as ("v" or "a", number)."""
+    out = set()
+    for kind, lo, hi, one in re.findall(r"\b([va])(?:\[(\d+):(\d+)\]|(\d+)\b)", text):
+        out.update((kind, n) for n in (range(int(lo), int(hi) + 1) if lo else [int(one)]))
+    return out
+
+
+def test_no_register_is_touched_while_an_lds_read_is_on_its_way_into_it(objects):
+    """The LDS reads of these kernels are inline assembly, whose latency the
+    compiler does not see: a copy or a spill of such a register that it places
+    ahead of the kernel's own lgkmcnt wait would take the value of before."""
+    reads = 0
+    for name, ins in _instructions(objects, "gemm_f32_split|gemm_ring|gemm_pers"):
+        pending = []  # one set of registers per LDS (or scalar) operation in flight, oldest first
+        for i in ins:
+            op, _, args = i.partition(" ")
+            wait = re.search(r"lgkmcnt\((\d+)\)", i) if op == "s_waitcnt" else None
+            if wait:
+                n = int(wait.group(1))
+                pending = pending[-n:] if n else []
+            elif op in ("s_branch", "s_endpgm"):
+                pending = []
+            elif pending:
+                busy = _registers(args) & set().union(*pending)
+                assert not busy, (name, i, busy)
+            if op.startswith("ds_read"):
+                reads += 1
+                pending.append(_registers(args.split(", v")[0]))
+            elif op.startswith(("ds_", "s_load", "s_buffer_load")):
+                pending.append(set())
+    assert reads > 1000
+
+
+def test_ring_and_split_kernels_spill_no_vector_register(objects):
+    """A spill is memory traffic in the loops whose DMA waits are counted by
+    hand, and a chance for the compiler to store a register too early (above)."""
+    seen = 0
+    for _, notes, _ in objects:
+        for block in re.split(r"\n  - \.agpr_count:", notes)[1:]:
+            name = re.search(r"\.name:\s+(_Z\w+)\n", block).group(1)
+            if re.search("gemm_f32_split|gemm_ring|gemm_pers|gemm_unaligned", name):
+                seen += 1
+                assert re.search(r"\.vgpr_spill_count: 0\n", block), name
+                assert re.search(r"\.private_segment_fixed_size: 0\n", block), name
+    assert seen > 50
