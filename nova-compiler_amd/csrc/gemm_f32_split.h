@@ -43,11 +43,19 @@
 // halves, eight k-lines apart, fall on different banks.  Rows need only be
 // 4-byte aligned.
 //
-// Range.  A value beyond the largest bf16 splits into infinity and NaN, and
-// one below 2^-109 has bits under the smallest bf16.  A wave whose outputs
-// are not all finite, or of which one is non-zero but below 2^-96, computes
-// its tile again on v_mfma_f32_32x32x2_f32 straight from memory: infinities,
-// NaNs, overflow and underflow come out as f32 arithmetic gives them.
+// Range.  Every value is split times 2^24, so that the lowest bit of the
+// smallest f32 subnormal, 2^-149, is a normal bf16's (and nothing depends on
+// how the MFMA takes subnormal inputs), and outputs are scaled back by 2^-48:
+// exact, and the same bits as without for ordinary operands.  A partial
+// product or sum too small for the accumulator is then below 2^-173 of the
+// output, under the smallest subnormal.  What is too large instead, an operand
+// from 2^104 on (its first piece is infinite and the next one NaN, whatever
+// it multiplies; infinities and NaNs likewise) or a sum from 2^80 on, leaves
+// outputs that are not finite: a wave computes such a block of its columns
+// again on v_mfma_f32_32x32x2_f32 straight from memory, so that infinities,
+// NaNs and overflow come out as f32 arithmetic gives them.  That costs the
+// blocks it happens to more than twice their time: 8192 x 8192 x 384 takes 408
+// us, 413 with a NaN in one row and 952 of nothing but NaNs.
 #pragma once
 
 #include "gemm_ring.h"
@@ -93,14 +101,17 @@ __device__ __forceinline__ float flip(float x, uint32_t sign) {
   return __uint_as_float(__float_as_uint(x) ^ sign);
 }
 
+constexpr float kUp = 0x1p24f, kDown = 0x1p-48f;  // see Range, at the top
+
 // Half of the splitting of values 2 q and 2 q + 1: h and the remainder
 // (unit 0), then m and l (unit 1).  FLIP: of the values with `sign` changed.
 template <bool FLIP>
 __device__ __forceinline__ void split_unit(Pieces &p, Raw &r, int q, int unit, uint32_t sign) {
   float a = r.v[q >> 1][2 * (q & 1)], b = r.v[q >> 1][2 * (q & 1) + 1];
-  if (FLIP && unit == 0) {
-    a = flip(a, sign);
-    b = flip(b, sign);
+  if (unit == 0) {
+    const float up = FLIP ? flip(kUp, sign) : kUp;
+    a = a * up;
+    b = b * up;
   }
   const uint32_t w = pack_bf16(a, b);
   a = a - __uint_as_float(w << 16);
@@ -221,10 +232,32 @@ __device__ __forceinline__ f32x16 mfma_bf16(u32x4 a, u32x4 b, f32x16 c) {
 __device__ __forceinline__ void dma16(const float *p, uint32_t bytes, char *base, uint32_t off) {
   ring::dma16(reinterpret_cast<const uint16_t *>(p), bytes, base, off);
 }
-__device__ __forceinline__ float load_f32(const float *p, uint32_t bytes, uint32_t off) {
-  return __builtin_bit_cast(
-      float, __builtin_amdgcn_raw_buffer_load_b32(
-                 make_rsrc(reinterpret_cast<const uint16_t *>(p), bytes), off, 0, 0));
+// Sixteen consecutive k of an operand's row straight from memory: zero where the
+// row is past the matrix (not `row_ok`) and from kend on, except that a
+// K-contiguous row's last chunk of four may go on into the next row.  (Offsets
+// of what is read are below 2^31, so 32 bits of them do.)
+template <bool KC>
+__device__ __forceinline__ void load_row(float (&v)[16], const float *p, uint32_t bytes, bool row_ok,
+                                         int row, uint32_t s_bytes, int k, int kend) {
+  const __amdgpu_buffer_rsrc_t rsrc = make_rsrc(reinterpret_cast<const uint16_t *>(p), bytes);
+  if constexpr (KC) {
+    const uint32_t off = (uint32_t)row * s_bytes + (uint32_t)k * 4u;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const f32x4 q = __builtin_bit_cast(
+          f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                     rsrc, row_ok && k + 4 * c < kend ? off + 16u * c : kOOB, 0, 0));
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[4 * c + e] = q[e];
+    }
+  } else {
+    const uint32_t off = (uint32_t)k * s_bytes + (uint32_t)row * 4u;
+#pragma unroll
+    for (int e = 0; e < 16; ++e)
+      v[e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                           rsrc, row_ok && k + e < kend ? off + e * s_bytes : kOOB,
+                                           0, 0));
+  }
 }
 
 // One unit of work: an output tile and the K steps [kt0, kt1) summed into it
@@ -515,72 +548,10 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_split_kernel(SplitArgs a) {
     }
     __builtin_amdgcn_sched_barrier(0);
 
-    // Outputs that the split does not represent: again in f32 (see the top).
-    // x * 0 is 0 or NaN; (x << 1) - 1 as an unsigned number orders by
-    // magnitude with zero on top.
-    // Values past the matrix's edges (whatever lies in memory there) do not
-    // count.
-    float fin = 0.0f;
-    uint32_t low = 0xffffffffu;
-    auto look = [&](float x) __attribute__((always_inline)) {
-      fin = __builtin_fmaf(x, 0.0f, fin);
-      low = min(low, (__float_as_uint(x) << 1) - 1u);
-    };
-    if (tc.m0 + BM <= a.M && tc.n0 + BN <= a.N) {
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-          for (int v = 0; v < 16; ++v) look(acc[i][j][v]);
-    } else {
-      const int rows = a.M - tc.m0 - am - (lane & 31), cols = a.N - tc.n0 - bn - 4 * (lane >> 5);
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-          for (int v = 0; v < 16; ++v)
-            look(32 * i < rows && 32 * j + 8 * (v >> 2) + (v & 3) < cols ? acc[i][j][v] : 0.0f);
-    }
-    constexpr uint32_t kTiny = (127u - 96u) << 24;  // 2^-96, shifted left by one
-    uint32_t sign = tc.sign;
-    if (__any(!(fin == 0.0f) || low < kTiny - 1u)) {
-      const float *Ab = a.A + (int64_t)tc.bidx * a.sab, *Bb = a.B + (int64_t)tc.bidx * a.sbb;
-      const int l32 = lane & 31, h = lane >> 5, kend = min(a.K, tc.kt1 * BK);
-      sign = 0;
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-          for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
-#pragma unroll 1
-      for (int k0 = tc.kt0 * BK; k0 < kend; k0 += 2) {
-        const int k = k0 + h;
-        float fa[TM], fb[TN];
-#pragma unroll
-        for (int i = 0; i < TM; ++i) {
-          const int64_t m = tc.m0 + am + 32 * i + l32;
-          fa[i] = load_f32(Ab, a.a_bytes, k < kend && m < a.M
-              ? (uint32_t)((AKC ? m * a.sa_outer + k : k * a.sa_outer + m) * 4) : kOOB);
-        }
-#pragma unroll
-        for (int j = 0; j < TN; ++j) {
-          const int64_t n = tc.n0 + bn + 32 * j + l32;
-          fb[j] = load_f32(Bb, a.b_bytes, k < kend && n < a.N
-              ? (uint32_t)((BKC ? n * a.sb_outer + k : k * a.sb_outer + n) * 4) : kOOB);
-        }
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-          for (int j = 0; j < TN; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fb[j], fa[i], acc[i][j], 0, 0, 0);
-      }
-    }
-
-    // Outputs straight from the accumulators: lane l holds columns
-    // 8 g + 4 (l / 32) ... + 3 of row l % 32 of a block, 16 bytes.
+    // Outputs straight from the accumulators, one column block at a time: lane
+    // l holds columns 8 g + 4 (l / 32) ... + 3 of row l % 32 of a block, 16
+    // bytes.  (The lane is opaque here: what is computed from it below is not
+    // kept in registers through the K loops.)
     const bool has_bias =
         (a.epi == NOVA_HIP_EPI_BIAS || a.epi == NOVA_HIP_EPI_BIAS_GELU) && tc.kt0 == 0;
     const bool has_gelu = (a.epi == NOVA_HIP_EPI_BIAS_GELU || a.epi == NOVA_HIP_EPI_GELU) &&
@@ -588,14 +559,10 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_split_kernel(SplitArgs a) {
     float *Cb = a.part ? a.part + ((int64_t)tc.split * a.batch + tc.bidx) * a.M * a.N
                        : a.C + (int64_t)tc.bidx * a.scb;
     const int64_t ldc = a.part ? a.N : a.scm;
-    const int lr = lane & 31, lh = lane >> 5;
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
+    int lr = lane & 31, lh = lane >> 5;
+    asm volatile("" : "+v"(lr), "+v"(lh));
+    auto store_column = [&](int j, f32x16 (&x)[TM]) __attribute__((always_inline)) {
       const int n = tc.n0 + bn + 32 * j + 4 * lh;
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) acc[i][j][v] = flip(acc[i][j][v], sign);
       if (has_bias) {
 #pragma unroll
         for (int g = 0; g < 4; ++g)
@@ -603,7 +570,7 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_split_kernel(SplitArgs a) {
           for (int e = 0; e < 4; ++e) {
             const float b = n + 8 * g + e < a.N ? bias_at(a.bias, a.bias_dt, n + 8 * g + e) : 0.0f;
 #pragma unroll
-            for (int i = 0; i < TM; ++i) acc[i][j][4 * g + e] += b;
+            for (int i = 0; i < TM; ++i) x[i][4 * g + e] += b;
           }
       }
 #pragma unroll
@@ -617,11 +584,11 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_split_kernel(SplitArgs a) {
             if (c + 4 <= a.N) {
               const f32x4 old = *reinterpret_cast<const f32x4u *>(row + c);
 #pragma unroll
-              for (int e = 0; e < 4; ++e) acc[i][j][4 * g + e] += old[e];
+              for (int e = 0; e < 4; ++e) x[i][4 * g + e] += old[e];
             } else {
 #pragma unroll
               for (int e = 0; e < 3; ++e)
-                if (c + e < a.N) acc[i][j][4 * g + e] += row[c + e];
+                if (c + e < a.N) x[i][4 * g + e] += row[c + e];
             }
           }
         }
@@ -629,35 +596,99 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_split_kernel(SplitArgs a) {
           f32x4 *blk = gelu_s[wave];
 #pragma unroll
           for (int g = 0; g < 4; ++g)
-            blk[g * 64 + lane] = f32x4{acc[i][j][4 * g], acc[i][j][4 * g + 1],
-                                       acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
+            blk[g * 64 + lane] = f32x4{x[i][4 * g], x[i][4 * g + 1], x[i][4 * g + 2], x[i][4 * g + 3]};
 #pragma unroll 1
           for (int g = 0; g < 4; ++g) {
-            f32x4 x = blk[g * 64 + lane];
+            f32x4 y = blk[g * 64 + lane];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) x[e] = gelu_tanh(x[e]);
-            blk[g * 64 + lane] = x;
+            for (int e = 0; e < 4; ++e) y[e] = gelu_tanh(y[e]);
+            blk[g * 64 + lane] = y;
           }
 #pragma unroll
           for (int g = 0; g < 4; ++g) {
-            const f32x4 x = blk[g * 64 + lane];
+            const f32x4 y = blk[g * 64 + lane];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) acc[i][j][4 * g + e] = x[e];
+            for (int e = 0; e < 4; ++e) x[i][4 * g + e] = y[e];
           }
         }
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
           const int c = n + 8 * g;
           if (m < a.M && c + 4 <= a.N) {
-            *reinterpret_cast<f32x4u *>(row + c) = f32x4{acc[i][j][4 * g], acc[i][j][4 * g + 1],
-                                                         acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
+            *reinterpret_cast<f32x4u *>(row + c) =
+                f32x4{x[i][4 * g], x[i][4 * g + 1], x[i][4 * g + 2], x[i][4 * g + 3]};
           } else if (m < a.M) {
 #pragma unroll
             for (int e = 0; e < 3; ++e)
-              if (c + e < a.N) row[c + e] = acc[i][j][4 * g + e];
+              if (c + e < a.N) row[c + e] = x[i][4 * g + e];
           }
         }
       }
+    };
+    // Values that are not finite keep their column block back for the loop
+    // below (see Range, at the top).  Those past the matrix's edges, where
+    // whatever lies in memory was multiplied, do not count.
+    const float down = flip(kDown, tc.sign);
+    uint32_t again = 0;
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      f32x16 x[TM];
+      float fin = 0.0f;  // x * 0 is 0 or NaN
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          x[i][v] = acc[i][j][v] * down;
+          fin = __builtin_fmaf(x[i][v], 0.0f, fin);
+        }
+      bool bad = __any(!(fin == 0.0f));
+      if (bad) {
+        const int n = tc.n0 + bn + 32 * j + 4 * lh;
+        fin = 0.0f;
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int v = 0; v < 16; ++v)
+            if (tc.m0 + am + 32 * i + lr < a.M && n + 8 * (v >> 2) + (v & 3) < a.N)
+              fin = __builtin_fmaf(x[i][v], 0.0f, fin);
+        bad = __any(!(fin == 0.0f));
+      }
+      if (bad) again |= 1u << j;
+      else store_column(j, x);
+    }
+    // Column blocks in f32 from memory, a whole 128-byte line of K-contiguous
+    // rows per step: lane half h takes the sixteen k from 16 h on.
+#pragma unroll 1
+    for (; again; again &= again - 1) {
+      const int j = __builtin_ctz(again);
+      const float *Ab = a.A + (int64_t)tc.bidx * a.sab, *Bb = a.B + (int64_t)tc.bidx * a.sbb;
+      const int kend = min(a.K, tc.kt1 * BK), n = tc.n0 + bn + 32 * j + lr;
+      f32x16 x[TM];
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) x[i][v] = 0.0f;
+#pragma unroll 1
+      for (int k = tc.kt0 * BK + 16 * lh; k - 16 * lh < kend; k += 32) {
+        float fa[TM][16], fb[16];
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+          const int m = tc.m0 + am + 32 * i + lr;
+          load_row<AKC>(fa[i], Ab, a.a_bytes, m < a.M, m, row_a, k, kend);
+        }
+        load_row<BKC>(fb, Bb, a.b_bytes, n < a.N, n, row_b, k, kend);
+        __builtin_amdgcn_sched_barrier(0);  // else each load sinks to its use and is waited for alone
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          // In a K-contiguous row the values from kend on are the next row's.
+          const float b = !BKC || k + e < kend ? fb[e] : 0.0f;
+#pragma unroll
+          for (int i = 0; i < TM; ++i)
+            x[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(
+                b, !AKC || k + e < kend ? fa[i][e] : 0.0f, x[i], 0, 0, 0);
+        }
+      }
+      store_column(j, x);
     }
     tc = next.t;
   }

@@ -71,8 +71,7 @@ def test_split_represents_every_f32(cuda, layout, flip):
 @pytest.mark.parametrize("scale", [1e-25, 1.0, 1e12])
 def test_split_error_bound(cuda, shape, scale):
     """Each output within (K / 2 + 8) 2^-24 of sum |a| |b|: the bound of an f32
-    accumulation of pairs, whatever the magnitude of the operands (1e-25 times
-    1e-3 products reach the f32 recomputation)."""
+    accumulation of pairs, whatever the magnitude of the operands."""
     import torch
     M, N, K = shape
     g = torch.Generator().manual_seed(M)
@@ -81,6 +80,34 @@ def test_split_error_bound(cuda, shape, scale):
     got = nh.gemm(A, B, f32_mfma=True).double()
     bound = (K / 2 + 8) * 2.0 ** -24 * torch.matmul(A.double().abs(), B.double().abs())
     assert bool(((got - torch.matmul(A.double(), B.double())).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("layout", LAYOUTS)
+@pytest.mark.parametrize("flip", [False, True])
+@pytest.mark.parametrize("K", [64, 1030])
+def test_split_operands_of_any_magnitude(cuda, layout, flip, K):
+    """Operands down to the smallest subnormal against ones that bring the
+    products back (2^-118 to 2^-149 times 2^80 to 2^120, one magnitude per row),
+    sums past what the split's own range holds (2^90), and products under the
+    smallest subnormal.  Each output within the bound of an f32 accumulation of
+    pairs, plus half the smallest subnormal for each product and each sum."""
+    import torch
+    g = torch.Generator().manual_seed(5)
+    M, N = 150, 70
+    rows = torch.tensor([-118, -122, -125, -126, -130, -140, -148, -20, 30, 0.0])
+    A = torch.randn(M, K, generator=g).double() * torch.exp2(rows.double())[torch.arange(M) % 10, None]
+    A[17], A[140] = 0.0, -0.0
+    cols = torch.tensor([120, 100, 80, 60, -30, -129, 0.0])
+    B = torch.randn(K, N, generator=g).double() * torch.exp2(cols.double())[None, torch.arange(N) % 7]
+    A, B = A.float(), B.float()
+    a, b = (B.t().contiguous(), A.t().contiguous()) if flip else (A, B)
+    C = nh.gemm(_lay(a.to(cuda), layout[0]), _lay(b.to(cuda), layout[1]), f32_mfma=True).cpu()
+    C = (C.t() if flip else C).double()
+    ref, scale = A.double() @ B.double(), A.double().abs() @ B.double().abs()
+    finite = scale < 3.4e38  # no sum of some of the products overflows
+    bound = (K / 2 + 8) * 2.0 ** -24 * scale + K * 2.0 ** -149
+    assert bool(((C - ref).abs() <= bound)[finite].all())
+    assert not bool(torch.isfinite(C[ref.abs() > 3.5e38]).any())
 
 
 @pytest.mark.parametrize("K", [100, 4100])
