@@ -638,7 +638,8 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_split_kernel(SplitArgs a) {
       for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
-          x[i][v] = acc[i][j][v] * down;
+          // (+ 0: a zero sum is +0 whichever sign was summed, as in f32.)
+          x[i][v] = __builtin_fmaf(acc[i][j][v], down, 0.0f);
           fin = __builtin_fmaf(x[i][v], 0.0f, fin);
         }
       bool bad = __any(!(fin == 0.0f));

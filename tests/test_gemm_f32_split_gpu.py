@@ -110,6 +110,21 @@ def test_split_operands_of_any_magnitude(cuda, layout, flip, K):
     assert not bool(torch.isfinite(C[ref.abs() > 3.5e38]).any())
 
 
+@pytest.mark.parametrize("shape", [(300, 260, 40), (300, 260, 0), (2100, 1900, 64), (130, 140, 2100)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_split_zero_sums_are_positive(cuda, shape):
+    """Sums of zeros of either sign and sums that cancel are +0 in every tile."""
+    import torch
+    M, N, K = shape
+    A = torch.zeros(M, K, device=cuda)
+    B = torch.ones(K, N, device=cuda)
+    A[::3] = -0.0
+    A[1::3, ::2], A[1::3, 1::2] = 1.5, -1.5
+    A[1::3, K // 2 * 2:] = 0.0
+    C = nh.gemm(A, B, f32_mfma=True)
+    assert bool((C == 0).all()) and not bool(torch.signbit(C).any())
+
+
 @pytest.mark.parametrize("K", [100, 4100])
 def test_split_operands_inside_larger_tensors(cuda, K):
     """Rows with odd strides at odd offsets, infinities all around: nothing
