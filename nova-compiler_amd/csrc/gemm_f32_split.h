@@ -232,31 +232,31 @@ __device__ __forceinline__ f32x16 mfma_bf16(u32x4 a, u32x4 b, f32x16 c) {
 __device__ __forceinline__ void dma16(const float *p, uint32_t bytes, char *base, uint32_t off) {
   ring::dma16(reinterpret_cast<const uint16_t *>(p), bytes, base, off);
 }
-// Sixteen consecutive k of an operand's row straight from memory: zero where the
-// row is past the matrix (not `row_ok`) and from kend on, except that a
-// K-contiguous row's last chunk of four may go on into the next row.  (Offsets
-// of what is read are below 2^31, so 32 bits of them do.)
+// Sixteen consecutive k of an operand's row straight from memory, the first
+// `left` of them: zero beyond, except that a K-contiguous row's last chunk of
+// four may go on into the next row.  (Offsets of what is read are below 2^31;
+// a negative left - 1 - e sets the bit that takes the others out of range.)
 template <bool KC>
-__device__ __forceinline__ void load_row(float (&v)[16], const float *p, uint32_t bytes, bool row_ok,
-                                         int row, uint32_t s_bytes, int k, int kend) {
+__device__ __forceinline__ void load_row(float (&v)[16], const float *p, uint32_t bytes, int left,
+                                         uint32_t row, uint32_t s_bytes, uint32_t k) {
   const __amdgpu_buffer_rsrc_t rsrc = make_rsrc(reinterpret_cast<const uint16_t *>(p), bytes);
+  auto at = [&](uint32_t off, int e) __attribute__((always_inline)) {
+    return off | ((uint32_t)(left - 1 - e) & kOOB);
+  };
   if constexpr (KC) {
-    const uint32_t off = (uint32_t)row * s_bytes + (uint32_t)k * 4u;
+    const uint32_t off = row * s_bytes + k * 4u;
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
       const f32x4 q = __builtin_bit_cast(
-          f32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                     rsrc, row_ok && k + 4 * c < kend ? off + 16u * c : kOOB, 0, 0));
+          f32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, at(off + 16u * c, 4 * c), 0, 0));
 #pragma unroll
       for (int e = 0; e < 4; ++e) v[4 * c + e] = q[e];
     }
   } else {
-    const uint32_t off = (uint32_t)k * s_bytes + (uint32_t)row * 4u;
+    uint32_t off = k * s_bytes + row * 4u;
 #pragma unroll
-    for (int e = 0; e < 16; ++e)
-      v[e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
-                                           rsrc, row_ok && k + e < kend ? off + e * s_bytes : kOOB,
-                                           0, 0));
+    for (int e = 0; e < 16; ++e, off += s_bytes)
+      v[e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, at(off, e), 0, 0));
   }
 }
 
@@ -307,8 +307,8 @@ typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 // before this one's outputs are written.  With more than one unit per
 // workgroup every unit has more than S steps (the steps being fetched when a
 // unit ends are then the next one's).
-template <bool AKC, bool BKC, int TM, int TN, int S>
-__global__ __launch_bounds__(kThreads) void gemm_f32_split_kernel(SplitArgs a) {
+template <bool AKC, bool BKC, int TM, int TN, int S, int PER_CU>
+__global__ __launch_bounds__(kThreads, PER_CU) void gemm_f32_split_kernel(SplitArgs a) {
   constexpr int BM = 64 * TM, BN = 64 * TN;
   constexpr int LA = 2 * TM, LB = 2 * TN, L = LA + LB;
   constexpr int kStageA = BM * BK * 4, kStage = (BM + BN) * BK * 4;
@@ -317,7 +317,9 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_split_kernel(SplitArgs a) {
   static_assert((S - 1) * L < 64, "vmcnt range");
 
   __shared__ __attribute__((aligned(128))) char smem[S * kStage];
-  __shared__ f32x4 gelu_s[4][256];  // one 32 x 32 block per wave
+  // One 32 x 32 block per wave; the smallest tile's one block fits registers.
+  constexpr bool kGeluLds = TM * TN > 1;
+  __shared__ f32x4 gelu_s[kGeluLds ? 4 : 1][kGeluLds ? 256 : 1];
   static_assert(sizeof(smem) + sizeof(gelu_s) <= 160 * 1024, "LDS");
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -592,7 +594,11 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_split_kernel(SplitArgs a) {
             }
           }
         }
-        if (has_gelu) {  // tanhf is large: in a rolled loop, through LDS
+        if (has_gelu && !kGeluLds) {
+#pragma unroll
+          for (int v = 0; v < 16; ++v) x[i][v] = gelu_tanh(x[i][v]);
+        }
+        if (has_gelu && kGeluLds) {  // tanhf is large: in a rolled loop, through LDS
           f32x4 *blk = gelu_s[wave];
 #pragma unroll
           for (int g = 0; g < 4; ++g)
@@ -662,6 +668,11 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_split_kernel(SplitArgs a) {
 #pragma unroll 1
     for (; again; again &= again - 1) {
       const int j = __builtin_ctz(again);
+      // (Opaque: what the loop makes of them is not worked out, and spilled,
+      // ahead of all units.)
+      uint32_t sa = row_a, sb = row_b;
+      int ml = tc.m0 + am;
+      asm volatile("" : "+s"(sa), "+s"(sb), "+s"(ml));
       const float *Ab = a.A + (int64_t)tc.bidx * a.sab, *Bb = a.B + (int64_t)tc.bidx * a.sbb;
       const int kend = min(a.K, tc.kt1 * BK), n = tc.n0 + bn + 32 * j + lr;
       f32x16 x[TM];
@@ -674,19 +685,20 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_split_kernel(SplitArgs a) {
         float fa[TM][16], fb[16];
 #pragma unroll
         for (int i = 0; i < TM; ++i) {
-          const int m = tc.m0 + am + 32 * i + lr;
-          load_row<AKC>(fa[i], Ab, a.a_bytes, m < a.M, m, row_a, k, kend);
+          const int m = ml + 32 * i + lr;
+          load_row<AKC>(fa[i], Ab, a.a_bytes, m < a.M ? kend - k : 0, m, sa, k);
         }
-        load_row<BKC>(fb, Bb, a.b_bytes, n < a.N, n, row_b, k, kend);
+        load_row<BKC>(fb, Bb, a.b_bytes, n < a.N ? kend - k : 0, n, sb, k);
         __builtin_amdgcn_sched_barrier(0);  // else each load sinks to its use and is waited for alone
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
           // In a K-contiguous row the values from kend on are the next row's.
-          const float b = !BKC || k + e < kend ? fb[e] : 0.0f;
+          const uint32_t in = ~(uint32_t)((kend - k - 1 - e) >> 31);
+          const float b = BKC ? __uint_as_float(__float_as_uint(fb[e]) & in) : fb[e];
 #pragma unroll
           for (int i = 0; i < TM; ++i)
             x[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(
-                b, !AKC || k + e < kend ? fa[i][e] : 0.0f, x[i], 0, 0, 0);
+                b, AKC ? __uint_as_float(__float_as_uint(fa[i][e]) & in) : fa[i][e], x[i], 0, 0, 0);
         }
       }
       store_column(j, x);
@@ -697,7 +709,10 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_split_kernel(SplitArgs a) {
 }
 
 // The tile forms (launch_form's cases, in this order) and what the choice
-// between them (gemm_f32_mfma.hip) needs to know of each.
+// between them (gemm_f32_mfma.hip) needs to know of each.  The workgroups per
+// CU are the kernel's last template argument too: its launch bound, which
+// keeps the registers of two 128 x 128 tiles within a CU's (206 each; 320
+// without).
 struct Form {
   int tm, tn, stages, per_cu;  // tile 64 tm x 64 tn; workgroups per CU
   float step, more, fixed;     // us: see estimate()
@@ -708,12 +723,12 @@ template <bool AKC, bool BKC>
 int32_t launch_form(int form, const SplitArgs &r, unsigned grid, hipStream_t s) {
   const dim3 g(grid), b(kThreads);
   switch (form) {
-    case 0: hipLaunchKernelGGL((gemm_f32_split_kernel<AKC, BKC, 4, 3, 2>), g, b, 0, s, r); break;
-    case 1: hipLaunchKernelGGL((gemm_f32_split_kernel<AKC, BKC, 3, 4, 2>), g, b, 0, s, r); break;
-    case 2: hipLaunchKernelGGL((gemm_f32_split_kernel<AKC, BKC, 3, 3, 2>), g, b, 0, s, r); break;
-    case 3: hipLaunchKernelGGL((gemm_f32_split_kernel<AKC, BKC, 4, 2, 2>), g, b, 0, s, r); break;
-    case 4: hipLaunchKernelGGL((gemm_f32_split_kernel<AKC, BKC, 2, 2, 2>), g, b, 0, s, r); break;
-    default: hipLaunchKernelGGL((gemm_f32_split_kernel<AKC, BKC, 1, 1, 3>), g, b, 0, s, r); break;
+    case 0: hipLaunchKernelGGL((gemm_f32_split_kernel<AKC, BKC, 4, 3, 2, 1>), g, b, 0, s, r); break;
+    case 1: hipLaunchKernelGGL((gemm_f32_split_kernel<AKC, BKC, 3, 4, 2, 1>), g, b, 0, s, r); break;
+    case 2: hipLaunchKernelGGL((gemm_f32_split_kernel<AKC, BKC, 3, 3, 2, 1>), g, b, 0, s, r); break;
+    case 3: hipLaunchKernelGGL((gemm_f32_split_kernel<AKC, BKC, 4, 2, 2, 1>), g, b, 0, s, r); break;
+    case 4: hipLaunchKernelGGL((gemm_f32_split_kernel<AKC, BKC, 2, 2, 2, 2>), g, b, 0, s, r); break;
+    default: hipLaunchKernelGGL((gemm_f32_split_kernel<AKC, BKC, 1, 1, 3, 3>), g, b, 0, s, r); break;
   }
   return check_hip(hipGetLastError(), "gemm_f32_split launch");
 }

@@ -88,15 +88,43 @@ def test_no_register_is_touched_while_an_lds_read_is_on_its_way_into_it(objects)
     assert reads > 1000
 
 
+def _resources(objects, pattern):
+    """(kernel, what its code object says of a resource) for each match."""
+    for _, notes, _ in objects:
+        for block in re.split(r"\n  - \.agpr_count:", notes)[1:]:
+            name = re.search(r"\.name:\s+(_Z\w+)\n", block).group(1)
+            if re.search(pattern, name):
+                yield name, lambda key: int(re.search(rf"\.{key}:\s+(\d+)\n", block).group(1))
+
+
 def test_ring_and_split_kernels_spill_no_vector_register(objects):
     """A spill is memory traffic in the loops whose DMA waits are counted by
     hand, and a chance for the compiler to store a register too early (above)."""
     seen = 0
-    for _, notes, _ in objects:
-        for block in re.split(r"\n  - \.agpr_count:", notes)[1:]:
-            name = re.search(r"\.name:\s+(_Z\w+)\n", block).group(1)
-            if re.search("gemm_f32_split|gemm_ring|gemm_pers|gemm_unaligned", name):
-                seen += 1
-                assert re.search(r"\.vgpr_spill_count: 0\n", block), name
-                assert re.search(r"\.private_segment_fixed_size: 0\n", block), name
+    for name, of in _resources(objects, "gemm_f32_split|gemm_ring|gemm_pers|gemm_unaligned"):
+        seen += 1
+        assert of("vgpr_spill_count") == 0 and of("private_segment_fixed_size") == 0, name
     assert seen > 50
+
+
+# Tile (64 TM x 64 TN, K groups) -> workgroups per CU that the choice of a form
+# and the tile order count on.
+PER_CU = {("ring", 4, 3, 1): 1, ("ring", 4, 2, 1): 1, ("ring", 2, 2, 2): 1, ("ring", 1, 2, 1): 2,
+          ("ring", 1, 1, 1): 3, ("ring", 1, 1, 2): 1,
+          ("f32_split", 4, 3, 1): 1, ("f32_split", 3, 4, 1): 1, ("f32_split", 3, 3, 1): 1,
+          ("f32_split", 4, 2, 1): 1, ("f32_split", 2, 2, 1): 2, ("f32_split", 1, 1, 1): 3}
+
+
+def test_as_many_workgroups_fit_a_cu_as_the_form_tables_say(objects):
+    """By LDS (160 KB) and by vector registers (512 per lane of a SIMD)."""
+    seen = 0
+    for name, of in _resources(objects, "gemm_f32_split|gemm_ring"):
+        kind = "ring" if "gemm_ring" in name else "f32_split"
+        tm, tn, _, *rest = map(int, re.findall(r"Li(\d+)E", name)[1 if kind == "ring" else 0:])
+        want = PER_CU[kind, tm, tn, rest[0] if kind == "ring" else 1]
+        waves = of("max_flat_workgroup_size") // 64 // 4  # per SIMD
+        registers = -(-of("vgpr_count") // 8) * 8
+        fit = min(160 * 1024 // of("group_segment_fixed_size"), 512 // registers // waves)
+        assert fit >= want, (name, fit, want)
+        seen += 1
+    assert seen == 72
