@@ -492,8 +492,9 @@ struct Form {
   int tm, tn, per_cu;  // tile 64 tm x 64 tn; workgroups that fit one CU's LDS
   int kg;
   float step, more, fixed;  // us: see choose()
+  int most;                 // K steps up to which it is considered
 };
-constexpr int kForms = 6;
+constexpr int kForms = 8;
 
 template <int DT>
 int32_t launch_form(int form, const RingArgs &r, bool akc, bool bkc, hipStream_t s) {
@@ -503,7 +504,9 @@ int32_t launch_form(int form, const RingArgs &r, bool akc, bool bkc, hipStream_t
     case 2: return launch_tile<DT, 2, 2, 2, 2>(r, akc, bkc, s);
     case 3: return launch_tile<DT, 1, 2, 3, 1>(r, akc, bkc, s);
     case 4: return launch_tile<DT, 1, 1, 3, 1>(r, akc, bkc, s);
-    default: return launch_tile<DT, 1, 1, 4, 2>(r, akc, bkc, s);
+    case 5: return launch_tile<DT, 1, 1, 4, 2>(r, akc, bkc, s);
+    case 6: return launch_tile<DT, 1, 1, 2, 1>(r, akc, bkc, s);
+    default: return launch_tile<DT, 1, 2, 2, 1>(r, akc, bkc, s);
   }
 }
 

@@ -7,27 +7,38 @@ namespace nova_hip {
 namespace ring {
 namespace {
 
-// Measured on one MI355X (bf16, all layouts, 56 shapes from 8 x 136 x 64 to
-// 4096^3, each on every form):
+// Measured on one MI355X (bf16, all layouts):
 //   step   time of one K step of a workgroup alone on its CU, chip full
 //   more   what each further workgroup on the CU adds to it
 //   fixed  a workgroup's launch, first loads and epilogue
-// With these, choose() lands within 1% of the best of these six forms (and
-// these six within 2.4% of the best of twelve) in the geometric mean.
+// The first six forms' constants are from 56 shapes, 8 x 136 x 64 to 4096^3,
+// each on every form.
+//
+// The last two are for short sums, where outputs and the first loads are the
+// time: two stages instead of three, so one less to fill and more workgroups
+// per CU.  Fitted, beside the others, to 220 shapes of K up to 512.  Against
+// the better of the same tiles with three stages they take 0.85 of the time at
+// one K step and more than three 64 x 64 tiles per CU (96 x [200 x 64] x
+// [64 x 200] 7.8 us, 9.7 with three; 2 x [1968 x 64] x [64 x 2656] 12.4 and
+// 13.9) and 0.87 at two; the gain goes down to 0.95 at eight steps, and from
+// 32 on they are behind (1.25 where a workgroup has its CU to itself).
+constexpr int kAny = 0x7fffffff;
 constexpr Form kForm[kForms] = {
-    {4, 3, 1, 1, 1.30f, 0.0f, 6.4f},    // 256 x 192: the least operand traffic
-    {4, 2, 1, 1, 0.926f, 0.0f, 4.7f},   // 256 x 128, three stages
-    {2, 2, 1, 2, 1.154f, 0.0f, 3.2f},   // 128 x 128, two K groups
-    {1, 2, 2, 1, 0.42f, 0.25f, 2.7f},   // 64 x 128
-    {1, 1, 3, 1, 0.30f, 0.12f, 2.7f},   // 64 x 64
-    {1, 1, 1, 2, 0.465f, 0.0f, 2.7f},   // 64 x 64, two K groups: few tiles
+    {4, 3, 1, 1, 1.30f, 0.0f, 6.4f, kAny},   // 256 x 192: the least operand traffic
+    {4, 2, 1, 1, 0.926f, 0.0f, 4.7f, kAny},  // 256 x 128, three stages
+    {2, 2, 1, 2, 1.154f, 0.0f, 3.2f, kAny},  // 128 x 128, two K groups
+    {1, 2, 2, 1, 0.42f, 0.25f, 2.7f, kAny},  // 64 x 128
+    {1, 1, 3, 1, 0.30f, 0.12f, 2.7f, kAny},  // 64 x 64
+    {1, 1, 1, 2, 0.465f, 0.0f, 2.7f, kAny},  // 64 x 64, two K groups: few tiles
+    {1, 1, 4, 1, 0.44f, 0.09f, 1.8f, 2},     // 64 x 64, two stages
+    {1, 2, 3, 1, 0.61f, 0.17f, 2.1f, 2},     // 64 x 128, two stages
 };
 // The persistent kernel's 256 x 256 tiles.  From a full round on it is the
 // faster one (4096^3: 114 us a round against 129 for 256 x 128); below, where
 // the ring's forms divide the chip badly (3072 x 4096 x 4096: 192 of its
 // tiles 102 us, 384 of 256 x 128 112 us), but not where they fit
 // (1024 x 11008 x 4096: 172 tiles 110 us, 232 of 256 x 192 88 us).
-constexpr Form kPersistent = {4, 4, 1, 1, 1.62f, 0.0f, 6.0f};
+constexpr Form kPersistent = {4, 4, 1, 1, 1.62f, 0.0f, 6.0f, kAny};
 
 int64_t tiles_of(const GemmArgs &a, const Form &f) {
   const int64_t bm = 64 * f.tm, bn = 64 * f.tn;
@@ -61,8 +72,9 @@ int choose(const GemmArgs &a, int cus) {
   int best = -1;
   float t = 0.0f;
   for (int i = 0; i < kForms + (whole ? 1 : 0); ++i) {
-    const float e = estimate(a, i < kForms ? kForm[i] : kPersistent, cus);
-    if (best < 0 || e < t) {
+    const Form &f = i < kForms ? kForm[i] : kPersistent;
+    const float e = estimate(a, f, cus);
+    if ((a.K + BK - 1) / BK <= f.most && (best < 0 || e < t)) {
       t = e;
       best = i;
     }

@@ -12,7 +12,8 @@ import nova_hip as nh
 
 pytestmark = pytest.mark.gpu
 
-# (batch, M, N, K, out): the form each is sized for.
+# (batch, M, N, K, out): the tile whose edges each is sized for.  (Which form runs
+# it is the estimate's choice; FORMS below reaches them all.)
 SHAPES = [
     (1, 1000, 3800, 136, "bf16"),    # 256 x 192, ragged last row and column
     (1, 1032, 11008, 328, "f32"),    # 256 x 192, one row group past a tile
@@ -25,7 +26,21 @@ SHAPES = [
     (1, 16, 1000, 1544, "bf16"),     # 64 x 64 in two K groups, 25 steps
     (1, 8, 8, 8, "f32"),             # one tile, one chunk of K: the second group has none
     (1, 64, 64, 64, "f16"),
-    (1, 72, 120, 0, "f32"),          # no K: zeros
+    (1, 72, 120, 0, "f32"),          # no K: zeros (A's rows 1 apart: the unaligned kernel's)
+]
+
+# One shape per form, by the smallest estimate: ragged in M, N and K.
+FORMS = [
+    (3, 200, 11008, 136, "bf16"),    # 256 x 192
+    (7, 2048, 264, 136, "f32"),      # 256 x 128
+    (1, 1500, 2056, 200, "f16"),     # 128 x 128 in two K groups
+    (2, 200, 2056, 136, "f32"),      # 64 x 128, three stages
+    (1, 200, 264, 136, "bf16"),      # 64 x 64, three stages
+    (1, 200, 264, 200, "f32"),       # 64 x 64 in two K groups
+    (1, 200, 264, 72, "f16"),        # 64 x 64, two stages
+    (2, 200, 8200, 72, "bf16"),      # 64 x 128, two stages
+    (2, 200, 8200, 128, "f32"),
+    (2, 256, 8200, 8, "f32"),
 ]
 
 
@@ -46,7 +61,7 @@ def _case(cuda, shape, layout, dt, seed):
 
 
 @pytest.mark.parametrize("layout", ["NN", "NT", "TN", "TT"])
-@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("shape", SHAPES + FORMS, ids=lambda s: "x".join(map(str, s)))
 def test_ring_exact(cuda, shape, layout):
     import torch
     for dt in ("bf16", "f16"):
@@ -110,3 +125,14 @@ def test_ring_values_beyond_k_do_not_leak(cuda):
 
         C = nh.gemm(embed(A), embed(B))
         assert torch.equal(C, ref.to(torch.float32)), layout
+
+
+def test_ring_without_k(cuda):
+    """K = 0 with rows that are 16-byte aligned: the epilogue of zeros."""
+    import torch
+    buf = torch.full((72 * 8,), float("nan"), device=cuda, dtype=torch.bfloat16)
+    bias = torch.randn(120, generator=torch.Generator().manual_seed(1)).to(cuda).to(torch.bfloat16)
+    A = buf.as_strided((1, 72, 0), (576, 8, 1))
+    B = torch.empty(1, 0, 120, device=cuda, dtype=torch.bfloat16)
+    C = nh.gemm(A, B, bias=bias, epilogue=nh.EPI_BIAS)
+    assert torch.equal(C[0], bias.float().expand(72, 120))

@@ -107,12 +107,13 @@ def test_ring_and_split_kernels_spill_no_vector_register(objects):
     assert seen > 50
 
 
-# Tile (64 TM x 64 TN, K groups) -> workgroups per CU that the choice of a form
-# and the tile order count on.
-PER_CU = {("ring", 4, 3, 1): 1, ("ring", 4, 2, 1): 1, ("ring", 2, 2, 2): 1, ("ring", 1, 2, 1): 2,
-          ("ring", 1, 1, 1): 3, ("ring", 1, 1, 2): 1,
-          ("f32_split", 4, 3, 1): 1, ("f32_split", 3, 4, 1): 1, ("f32_split", 3, 3, 1): 1,
-          ("f32_split", 4, 2, 1): 1, ("f32_split", 2, 2, 1): 2, ("f32_split", 1, 1, 1): 3}
+# Tile (64 TM x 64 TN), stages, K groups -> workgroups per CU that the choice of
+# a form and the tile order count on.
+PER_CU = {("ring", 4, 3, 2, 1): 1, ("ring", 4, 2, 3, 1): 1, ("ring", 2, 2, 2, 2): 1,
+          ("ring", 1, 2, 3, 1): 2, ("ring", 1, 1, 3, 1): 3, ("ring", 1, 1, 4, 2): 1,
+          ("ring", 1, 1, 2, 1): 4, ("ring", 1, 2, 2, 1): 3,
+          ("f32_split", 4, 3, 2, 1): 1, ("f32_split", 3, 4, 2, 1): 1, ("f32_split", 3, 3, 2, 1): 1,
+          ("f32_split", 4, 2, 2, 1): 1, ("f32_split", 2, 2, 2, 1): 2, ("f32_split", 1, 1, 3, 1): 3}
 
 
 def test_as_many_workgroups_fit_a_cu_as_the_form_tables_say(objects):
@@ -120,11 +121,11 @@ def test_as_many_workgroups_fit_a_cu_as_the_form_tables_say(objects):
     seen = 0
     for name, of in _resources(objects, "gemm_f32_split|gemm_ring"):
         kind = "ring" if "gemm_ring" in name else "f32_split"
-        tm, tn, _, *rest = map(int, re.findall(r"Li(\d+)E", name)[1 if kind == "ring" else 0:])
-        want = PER_CU[kind, tm, tn, rest[0] if kind == "ring" else 1]
+        tm, tn, stages, rest = map(int, re.findall(r"Li(\d+)E", name)[1 if kind == "ring" else 0:])
+        want = PER_CU[kind, tm, tn, stages, rest if kind == "ring" else 1]
         waves = of("max_flat_workgroup_size") // 64 // 4  # per SIMD
         registers = -(-of("vgpr_count") // 8) * 8
         fit = min(160 * 1024 // of("group_segment_fixed_size"), 512 // registers // waves)
         assert fit >= want, (name, fit, want)
         seen += 1
-    assert seen == 72
+    assert seen == 88
