@@ -136,23 +136,40 @@ typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 // beyond their own 4 bytes: 16-byte stores take any (element-by-element
 // stores of odd rows took 93.3 us where this takes 58.6 at 48x[997x64]x[64x997],
 // 59.5 against 50.6 at 4000x3002x1024; aligned rows the same either way).
-// f32 with GELU (tanhf is large) goes element by element in a rolled loop.
+// f32 with GELU (tanhf is large) goes two chunks at a time in a rolled loop.
 template <int ROWS, int COLS, int NT, int KG>
 __device__ __forceinline__ void store_f32(char *stg, int dist, int tid, float *C, int64_t ld,
                                           int rows, int cols, const float *bias, bool gelu) {
   constexpr int CR = COLS / 4, kIt = ROWS * CR / NT;  // 4-column chunks per row, per thread
   static_assert(ROWS * CR % NT == 0, "whole rounds");
+  // 16 bytes at once where the chunk is whole.
+  auto put = [&](int it, f32x4 x) __attribute__((always_inline)) {
+    const int q = it * NT + tid, R = q / CR, n = 4 * (q - R * CR);
+    if (R < rows && n + 4 <= cols) {
+      *reinterpret_cast<f32x4u *>(C + R * ld + n) = x;
+    } else if (R < rows) {
+#pragma unroll
+      for (int e = 0; e < 3; ++e)
+        if (n + e < cols) C[R * ld + n + e] = x[e];
+    }
+  };
   if (gelu) {
+    constexpr int kU = kIt % 2 == 0 ? 2 : 1;
 #pragma unroll 1
-    for (int it = 0; it < kIt; ++it) {
-      const int q = it * NT + tid, R = q / CR, c = q - R * CR;
-      f32x4 x = staged_sum<COLS, KG>(stg, dist, R, c);
-      if (bias) x = x + *reinterpret_cast<const f32x4 *>(bias + 4 * c);
+    for (int it = 0; it < kIt; it += kU) {
+      f32x4 x[kU];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) x[e] = gelu_tanh(x[e]);
+      for (int u = 0; u < kU; ++u) {
+        const int q = (it + u) * NT + tid, R = q / CR, c = q - R * CR;
+        x[u] = staged_sum<COLS, KG>(stg, dist, R, c);
+        if (bias) x[u] = x[u] + *reinterpret_cast<const f32x4 *>(bias + 4 * c);
+      }
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (R < rows && 4 * c + e < cols) C[R * ld + 4 * c + e] = x[e];
+      for (int u = 0; u < kU; ++u)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[u][e] = gelu_tanh(x[u][e]);
+#pragma unroll
+      for (int u = 0; u < kU; ++u) put(it + u, x[u]);
     }
     return;
   }
@@ -168,16 +185,7 @@ __device__ __forceinline__ void store_f32(char *stg, int dist, int tid, float *C
       x[it] = x[it] + *reinterpret_cast<const f32x4 *>(bias + 4 * ((it * NT + tid) % CR));
   }
 #pragma unroll
-  for (int it = 0; it < kIt; ++it) {
-    const int q = it * NT + tid, R = q / CR, n = 4 * (q - R * CR);
-    if (R < rows && n + 4 <= cols) {
-      *reinterpret_cast<f32x4u *>(C + R * ld + n) = x[it];
-    } else if (R < rows) {
-#pragma unroll
-      for (int e = 0; e < 3; ++e)
-        if (n + e < cols) C[R * ld + n + e] = x[it][e];
-    }
-  }
+  for (int it = 0; it < kIt; ++it) put(it, x[it]);
 }
 
 template <int ROWS, int COLS, int NT, int KG>

@@ -21,7 +21,8 @@ namespace {
 // one K step and more than three 64 x 64 tiles per CU (96 x [200 x 64] x
 // [64 x 200] 7.8 us, 9.7 with three; 2 x [1968 x 64] x [64 x 2656] 12.4 and
 // 13.9) and 0.87 at two; the gain goes down to 0.95 at eight steps, and from
-// 32 on they are behind (1.25 where a workgroup has its CU to itself).
+// 32 on they are behind (1.25 where a workgroup has its CU to itself).  With a
+// CU to each they gain nothing at any length, and are not considered.
 constexpr int kAny = 0x7fffffff;
 constexpr Form kForm[kForms] = {
     {4, 3, 1, 1, 1.30f, 0.0f, 6.4f, kAny},   // 256 x 192: the least operand traffic
@@ -49,21 +50,31 @@ int64_t tiles_of(const GemmArgs &a, const Form &f) {
 // steps.  A chip that is not full runs its steps faster (up to 30%: less
 // contention in L2, a higher clock), and so does the last, partial round;
 // where several workgroups share a CU the next tile starts as one ends, so
-// rounds need not be whole.
+// rounds need not be whole.  GELU of f32 outputs is tanhf on the ring kernel,
+// kGelu us for each output of a thread (192 of them in a 256 x 192 tile): with
+// it, 3434 x 1776 x 432 takes 43 us in that form and 20 in 64 x 64 tiles, which
+// several workgroups per CU share in time.  (The persistent kernel's GELU is
+// gelu_tanh_fast: a tenth.)
+constexpr float kGelu = 0.1f;
 float estimate(const GemmArgs &a, const Form &f, int cus) {
   const float q = (float)tiles_of(a, f) / cus;
   const int nk = (a.K + BK - 1) / BK, steps = (nk + f.kg - 1) / f.kg;
+  const float share = q <= 1.0f ? 1.0f : q <= f.per_cu ? ceilf(q) : f.per_cu;  // of a CU
+  const bool gelu = a.out_dt == NOVA_HIP_DT_F32 &&
+                    (a.epi == NOVA_HIP_EPI_BIAS_GELU || a.epi == NOVA_HIP_EPI_GELU);
+  const float fixed =
+      f.fixed + (gelu ? (&f == &kPersistent ? 0.1f : 1.0f) * kGelu * (16 * f.tm * f.tn / f.kg) : 0.0f);
   float step, rounds = 1.0f;
   if (q <= 1.0f) {
     step = f.step * (0.7f + 0.3f * q);
-  } else if (q <= f.per_cu) {
-    step = f.step + f.more * (ceilf(q) - 1.0f);
   } else {
-    step = f.step + f.more * (f.per_cu - 1);
+    step = f.step + f.more * (share - 1.0f);
+  }
+  if (q > f.per_cu) {
     const float r = q / f.per_cu, whole = floorf(r), part = r - whole;
     rounds = f.per_cu > 1 ? r + 0.25f : part > 0.0f ? whole + 0.7f + 0.3f * part : whole;
   }
-  return rounds * (steps * step + f.fixed);
+  return rounds * (steps * step + fixed);
 }
 
 // The form of least estimated time; kForms: the persistent kernel.
@@ -74,7 +85,8 @@ int choose(const GemmArgs &a, int cus) {
   for (int i = 0; i < kForms + (whole ? 1 : 0); ++i) {
     const Form &f = i < kForms ? kForm[i] : kPersistent;
     const float e = estimate(a, f, cus);
-    if ((a.K + BK - 1) / BK <= f.most && (best < 0 || e < t)) {
+    if (f.most < kAny && ((a.K + BK - 1) / BK > f.most || tiles_of(a, f) <= cus)) continue;
+    if (best < 0 || e < t) {
       t = e;
       best = i;
     }

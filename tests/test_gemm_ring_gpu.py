@@ -37,7 +37,7 @@ FORMS = [
     (2, 200, 2056, 136, "f32"),      # 64 x 128, three stages
     (1, 200, 264, 136, "bf16"),      # 64 x 64, three stages
     (1, 200, 264, 200, "f32"),       # 64 x 64 in two K groups
-    (1, 200, 264, 72, "f16"),        # 64 x 64, two stages
+    (20, 200, 264, 72, "f16"),       # 64 x 64, two stages
     (2, 200, 8200, 72, "bf16"),      # 64 x 128, two stages
     (2, 200, 8200, 128, "f32"),
     (2, 256, 8200, 8, "f32"),
