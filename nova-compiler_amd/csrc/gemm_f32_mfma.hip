@@ -145,25 +145,30 @@ int32_t launch_gemm_f32_mfma(const GemmProblem &p, hipStream_t s) {
 
   // The form and, when K is long enough to share, the number of splits (up
   // to 8 of at least 1024, their partials at most 1 GiB) of least estimated
-  // time.
+  // time.  A stream under capture whose workspace cannot hold the partials
+  // takes one split: which calls want several is this choice's affair.
   const int cus = device_cu_count() > 0 ? device_cu_count() : 256;
   const double out_bytes = (double)p.batch * p.M * p.N * 4.0;
+  const int64_t per_split = p.batch * p.M * p.N;
   int form = 0, splits = 1;
-  float best = 0.0f;
-  for (int f = 0; f < kForms; ++f)
-    for (int sp = 1; sp <= 8 && (sp == 1 || (p.K >= 2048 && p.K / sp >= 1024 &&
-                                             sp * out_bytes <= 1073741824.0));
-         ++sp) {
-      const float us = estimate(a, kForm[f], sp, cus);
-      if ((f == 0 && sp == 1) || us < best) {
-        best = us;
-        form = f;
-        splits = sp;
+  for (int most = 8;; most = 1) {
+    float best = 0.0f;
+    for (int f = 0; f < kForms; ++f)
+      for (int sp = 1; sp <= most && (sp == 1 || (p.K >= 2048 && p.K / sp >= 1024 &&
+                                                  sp * out_bytes <= 1073741824.0));
+           ++sp) {
+        const float us = estimate(a, kForm[f], sp, cus);
+        if ((f == 0 && sp == 1) || us < best) {
+          best = us;
+          form = f;
+          splits = sp;
+        }
       }
-    }
+    if (splits == 1 || !WorkspaceLease::refused_by_capture(s, (size_t)(splits * per_split) * 4)) break;
+  }
   const Form &f = kForm[form];
-  a.tiles_m = (a.M + 64 * f.tm - 1) / (64 * f.tm);
-  a.tiles_n = (a.N + 64 * f.tn - 1) / (64 * f.tn);
+  a.tiles_m = (int)((p.M + 64 * f.tm - 1) / (64 * f.tm));
+  a.tiles_n = (int)((p.N + 64 * f.tn - 1) / (64 * f.tn));
   a.splits = splits;
   const int nk = (a.K + BK - 1) / BK;
   a.chunks = chunks_of(a, splits);
@@ -177,7 +182,6 @@ int32_t launch_gemm_f32_mfma(const GemmProblem &p, hipStream_t s) {
   const int64_t grid =
       nk / (splits * a.chunks) > f.stages && units > cus * f.per_cu ? cus * f.per_cu : units;
 
-  const int64_t per_split = p.batch * p.M * p.N;
   WorkspaceLease lease;  // the partials, held until their reduction is enqueued
   if (splits > 1) {
     a.part = static_cast<float *>(lease.acquire(s, (size_t)(splits * per_split) * 4));

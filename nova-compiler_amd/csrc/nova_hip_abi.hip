@@ -123,6 +123,20 @@ void *WorkspaceLease::acquire(hipStream_t s, size_t bytes) {
   return ptr_;
 }
 
+bool WorkspaceLease::refused_by_capture(hipStream_t s, size_t bytes) {
+  {
+    std::lock_guard<std::mutex> lock(g_ws_mu);
+    const auto it = g_ws.find(s);
+    if (it != g_ws.end() && it->second.ptr && it->second.bytes >= bytes) return false;
+  }
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &status) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return status != hipStreamCaptureStatusNone;
+}
+
 namespace {
 
 // ---- descriptor helpers ----------------------------------------------------

@@ -190,6 +190,9 @@ class WorkspaceLease {
   WorkspaceLease &operator=(const WorkspaceLease &) = delete;
   void *acquire(hipStream_t s, size_t bytes);
   void *get() const { return ptr_; }
+  // Whether acquire() would have to allocate on a stream that is being
+  // captured into a graph, where it cannot.
+  static bool refused_by_capture(hipStream_t s, size_t bytes);
 
  private:
   std::unique_lock<std::mutex> lock_;

@@ -83,3 +83,32 @@ def test_library_calls_replay_from_a_hip_graph(cuda):
         torch.cuda.synchronize()
         for k, (a, e) in enumerate(zip(got, outs)):
             assert torch.equal(a, e), (i, k)
+
+
+def test_f32_gemm_of_a_long_sum_captures_on_a_stream_without_workspace(cuda):
+    """The matrix-core f32 GEMM whose K it would share out with partial sums in
+    the workspace takes one split where that would have to be allocated under
+    capture: every replay equals the product of its inputs (integers: exact in
+    any order)."""
+    import torch
+    M, N, K = 200, 300, 8192
+    g = torch.Generator().manual_seed(1)
+    A, B = torch.empty(M, K, device=cuda), torch.empty(K, N, device=cuda)
+    C = torch.empty(M, N, device=cuda)
+    s = torch.cuda.Stream()
+    nh.lib().nova_hip_release_workspace()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(s):
+        with torch.cuda.graph(graph, stream=s):
+            nh.gemm(A, B, C, f32_mfma=True)
+    torch.cuda.synchronize()
+    for _ in range(3):
+        A.copy_(torch.randint(-30, 31, (M, K), generator=g).float())
+        B.copy_(torch.randint(-9, 10, (K, N), generator=g).float())
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        ref = A.double() @ B.double()
+        assert torch.equal(C.double(), ref)
+        eager = nh.gemm(A, B, f32_mfma=True)  # in splits, on the current stream
+        assert torch.equal(eager.double(), ref)
