@@ -133,8 +133,9 @@ enum {
  * pieces, six of whose nine products are summed in f32 (the other three are
  * below 2^-26 of the product).  In the MFMA's and the tile loop's order, not
  * the reference's sequential k: the result is within the f32 parity bar (1e-4
- * relative), not bit-identical to Nova's CPU pipeline.  Same results on every run.  f32 in and out; the
- * epilogues as for the other kernels.  Also accepted by the backward GEMM
+ * relative) for operands of any magnitude, not bit-identical to Nova's CPU
+ * pipeline.  Same results on every run.  f32 in and out; the epilogues as for
+ * the other kernels.  Also accepted by the backward GEMM
  * entry points. */
 #define NOVA_HIP_GEMM_F32_MFMA 0x20000
 

@@ -13,9 +13,9 @@
 // the same on every run.
 //
 // Against v_mfma_f32_32x32x2_f32 in 128 x 128 tiles, us on one MI355X:
-// 8192 x 50304 x 384 2649 -> 1718, 8192 x 384 x 50304 2414 -> 1528,
-// 384 x 50304 x 8192 2543 -> 1613, 8192 x 1536 x 384 87 -> 57,
-// 1536 x 384 x 8192 146 -> 66, 256^3 24.1 -> 8.7.
+// 8192 x 50304 x 384 2649 -> 1678, 8192 x 384 x 50304 2414 -> 1549,
+// 384 x 50304 x 8192 2543 -> 1602, 8192 x 1536 x 384 87 -> 57,
+// 384 x 1536 x 8192 141 -> 69, 2000 x 50304 x 32 137 -> 124, 256^3 24.1 -> 10.0.
 #include "gemm_f32_split.h"
 
 namespace nova_hip {

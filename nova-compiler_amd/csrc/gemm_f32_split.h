@@ -31,7 +31,7 @@
 //
 // What bounds it: MFMA issue and the board's power limit.  A K step moves as
 // many bytes through LDS as a bf16 GEMM's and multiplies three times as long
-// on them, so two stages hide the DMA.  The splitting is VALU work (11
+// on them, so two stages hide the DMA.  The splitting is VALU work (13
 // operations per pair of values) beside the MFMAs of the step before: it is
 // done as fragments are read, once per wave that needs one, which is why the
 // wave tiles are as large as the registers allow.
@@ -46,16 +46,18 @@
 // Range.  Every value is split times 2^24, so that the lowest bit of the
 // smallest f32 subnormal, 2^-149, is a normal bf16's (and nothing depends on
 // how the MFMA takes subnormal inputs), and outputs are scaled back by 2^-48:
-// exact, and the same bits as without for ordinary operands.  A partial
-// product or sum too small for the accumulator is then below 2^-173 of the
-// output, under the smallest subnormal.  What is too large instead, an operand
+// exact but where an output is subnormal, and the same bits as without for
+// ordinary operands.  What is too small for the accumulator is then under
+// 2^-173 in the output, below the smallest subnormal.  What is too large, an operand
 // from 2^104 on (its first piece is infinite and the next one NaN, whatever
 // it multiplies; infinities and NaNs likewise) or a sum from 2^80 on, leaves
 // outputs that are not finite: a wave computes such a block of its columns
 // again on v_mfma_f32_32x32x2_f32 straight from memory, so that infinities,
 // NaNs and overflow come out as f32 arithmetic gives them.  That costs the
 // blocks it happens to more than twice their time: 8192 x 8192 x 384 takes 408
-// us, 413 with a NaN in one row and 952 of nothing but NaNs.
+// us, 413 with a NaN in one row and 952 of nothing but NaNs.  The scaling costs
+// nothing where the MFMAs are the bound, and up to 7% of the 64 x 64 form, whose
+// bound is the splitting (256^3 9.4 -> 10.0 us).
 #pragma once
 
 #include "gemm_ring.h"
